@@ -11,7 +11,7 @@
 // scheduling.
 
 #include "gemm_engine.hpp"
-#include "mfma_tile.hpp"
+#include "split_mma.hpp"
 #include "tune.hpp"
 #include "../../include/nert_hip.h"
 
@@ -20,67 +20,149 @@
 #include <array>
 #include <map>
 #include <mutex>
+#include <type_traits>
 
 namespace nert_hip {
 namespace {
 
-// Builds the loader of one operand. `row_stride`/`k_stride` are the element
-// strides of the operand's non-K and K index; K_CONTIG selects which is 1.
-template <int ROWS, int BK, int THREADS, int PITCH, bool K_CONTIG, bool CHECKED>
-__device__ __forceinline__ auto MakeOperand(const float* base, int64_t row0, int64_t row_stride, int64_t k_stride,
-                                            int64_t rows, int64_t k_total) {
-    if constexpr (K_CONTIG) {
-        KContigLoader<ROWS, BK, THREADS, PITCH, CHECKED> l;
-        l.base = base + row0 * row_stride;
-        l.row_stride = row_stride;
-        l.rows_left = rows - row0;
-        l.k_total = k_total;
-        return l;
-    } else {
-        RowContigLoader<ROWS, BK, THREADS, PITCH, CHECKED> l;
-        l.base = base + row0;
-        l.k_stride = k_stride;
-        l.rows_left = rows - row0;
-        l.k_total = k_total;
-        return l;
-    }
-}
+// One workgroup's tile: BM x BN outputs by WAVES_M x WAVES_N waves, K in steps
+// of 32 (one MFMA).
+template <int BM, int BN, int WAVES_M, int WAVES_N>
+struct GemmTile {
+    static constexpr int kBM = BM;
+    static constexpr int kBN = BN;
+    static constexpr int kBK = 32;
+    static constexpr int kWavesM = WAVES_M;
+    static constexpr int kThreads = 64 * WAVES_M * WAVES_N;
+    static constexpr int kRows = BM / WAVES_M; // per wave
+    static constexpr int kCols = BN / WAVES_N;
+    static constexpr int kRB = kRows / 16; // 16 x 16 blocks per wave
+    static constexpr int kCB = kCols / 16;
+    static_assert(kRows % 16 == 0 && kCols % 16 == 0, "wave tiles are whole 16 x 16 blocks");
+};
 
-// B of a patch convolution read in place (GemmArgs::PatchB): each thread
-// loads runs of 4 consecutive k of one column n, i.e. 4 consecutive input
-// columns of one input row, into the k-major LDS tile the way the
-// K-contiguous loader does. The x offsets of the thread's columns at k = 0
-// are fixed for the whole K walk; a k's offset is c * H * W + r * W + q.
-template <int ROWS, int BK, int THREADS, int PITCH, bool CHECKED>
-struct PatchLoader {
-    using Rows = KContigLoader<ROWS, BK, THREADS, PITCH, CHECKED>;
-    static constexpr int kQuads = Rows::kQuads;
-    static constexpr int kPer = Rows::kPer;
-    using Stage = typename Rows::Stage;
-    const GemmArgs::PatchB* v;
-    uint32_t col_off[kPer];
-    bool col_ok[kPer];
-    uint32_t k_total;
+// LDS form of one operand's K step: ROWS / 16 fragments per piece, a fragment
+// being 64 slots of 16 bytes in lane order (slot l: row l % 16, k octet
+// l / 16). An MFMA operand is then one ds_read_b128 of 64 consecutive slots,
+// and the stores below write 16 consecutive slots per 16 lanes: neither has
+// bank conflicts.
+template <int ROWS>
+constexpr int kOperandLds = ROWS * 48; // uint32 words: 3 pieces x 32 k x 2 bytes per row
 
-    __device__ __forceinline__ void init(const GemmArgs::PatchB& pv, int64_t col0, int64_t n_total, int64_t k_tot) {
-        v = &pv;
-        k_total = static_cast<uint32_t>(k_tot);
+// Four floats at any 4-byte address (global memory takes 16-byte loads there).
+typedef float UnalignedQuad __attribute__((ext_vector_type(4), aligned(4)));
+
+// Operand stagers: a thread owns kPer octets (8 consecutive k of one row) of
+// every K step, loads them to registers and later splits and stores them.
+//
+// K index contiguous (A row-major, B transposed, or a patch convolution's
+// input): octet q is row 16 * (q / 64) + q % 16, k octet q % 64 / 16, so the
+// four lanes of a row cover its 128 bytes.
+template <int ROWS, int THREADS>
+struct KOctets {
+    static constexpr int kPer = ROWS * 4 / THREADS;
+    static_assert(ROWS * 4 % THREADS == 0, "every thread owns the same number of octets");
+    static __device__ __forceinline__ int Row(int q) { return q / 64 * 16 + q % 16; }
+    static __device__ __forceinline__ int Oct(int q) { return q % 64 / 16; }
+    static __device__ __forceinline__ int Slot(int q) { return q; }
+};
+
+// Row index contiguous (A transposed, B row-major): octet q is row q % ROWS,
+// k octet q / ROWS, so a load of one k takes consecutive rows.
+template <int ROWS, int THREADS>
+struct RowOctets {
+    static constexpr int kPer = ROWS * 4 / THREADS;
+    static_assert(ROWS * 4 % THREADS == 0, "every thread owns the same number of octets");
+    static __device__ __forceinline__ int Row(int q) { return q % ROWS; }
+    static __device__ __forceinline__ int Oct(int q) { return q / ROWS; }
+    static __device__ __forceinline__ int Slot(int q) { return q % ROWS / 16 * 64 + q / ROWS * 16 + q % 16; }
+};
+
+// A strided operand: element (row, k) at base[row * row_stride + k * k_stride],
+// one of the strides 1. Rows past the operand repeat its last one (they only
+// reach outputs that are never stored). A thread's byte offsets from the
+// K step's base are fixed; `Offset` is 32 bits wide (scalar base plus vector
+// offset, no address arithmetic per load) unless the strides need 64.
+template <int ROWS, int THREADS, bool K_CONTIG, class Offset>
+struct StridedOperand {
+    using Map = std::conditional_t<K_CONTIG, KOctets<ROWS, THREADS>, RowOctets<ROWS, THREADS>>;
+    const float* base; // row 0 of the tile
+    int64_t row_stride;
+    int64_t k_stride;
+    int64_t last; // last valid row of the tile
+    Offset off[Map::kPer];
+
+    __device__ __forceinline__ void Init(const float* b, int64_t row0, int64_t rs, int64_t ks, int64_t total) {
+        base = b + row0 * rs;
+        row_stride = rs;
+        k_stride = ks;
+        last = total - 1 - row0;
 #pragma unroll
-        for (int p = 0; p < kPer; ++p) {
-            const int q = threadIdx.x + p * THREADS;
-            const int64_t n = col0 + q / (BK / 4);
-            col_ok[p] = q < kQuads && n < n_total;
-            // Columns past the operand (an edge tile) read its last column:
-            // they only feed outputs that are never stored.
-            const uint32_t nn = static_cast<uint32_t>(n < n_total ? n : n_total - 1);
-            uint32_t rem;
-            const uint32_t img = DivMod(pv.div_plane, nn, rem);
-            uint32_t ow;
-            const uint32_t oh = DivMod(pv.div_ow, rem, ow);
-            col_off[p] = ((img * static_cast<uint32_t>(pv.c) * static_cast<uint32_t>(pv.in_h) +
-                           oh * static_cast<uint32_t>(pv.kh)) *
-                              static_cast<uint32_t>(pv.in_w) +
-                          ow * static_cast<uint32_t>(pv.kw));
+        for (int p = 0; p < Map::kPer; ++p) {
+            const int q = static_cast<int>(threadIdx.x) + p * THREADS;
+            off[p] = static_cast<Offset>((RowAt(Map::Row(q)) + 8 * Map::Oct(q) * (K_CONTIG ? 1 : ks)) * 4);
+        }
+    }
+    __device__ __forceinline__ int64_t RowAt(int row) const {
+        const int64_t r = row < last ? row : last;
+        return K_CONTIG ? r * row_stride : r;
+    }
+    // Whether 32-bit offsets reach every element of a step of a tile.
+    static bool Narrow(int64_t rs, int64_t ks) {
+        return K_CONTIG ? rs < (int64_t{1} << 30) / ROWS - 32 : ks < (int64_t{1} << 30) / 32 - ROWS;
+    }
+    // A whole step (k0 + 32 within K).
+    __device__ __forceinline__ void LoadFull(int p, int64_t k0, nert_floatx4& lo, nert_floatx4& hi) const {
+        if constexpr (K_CONTIG) {
+            const char* at = reinterpret_cast<const char*>(base + k0) + off[p];
+            lo = *reinterpret_cast<const UnalignedQuad*>(at);
+            hi = *reinterpret_cast<const UnalignedQuad*>(at + 16);
+        } else {
+            float f[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                f[e] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base + (k0 + e) * k_stride) +
+                                                       off[p]);
+            }
+            lo = nert_floatx4{f[0], f[1], f[2], f[3]};
+            hi = nert_floatx4{f[4], f[5], f[6], f[7]};
+        }
+    }
+    __device__ __forceinline__ float At(int row, int64_t k) const {
+        return base[RowAt(row) + (K_CONTIG ? k : k * k_stride)];
+    }
+};
+
+// B of a patch convolution read in place (GemmArgs::PatchB): the x offsets of
+// the thread's columns at k = 0 are fixed for the whole K walk; a k's offset
+// is c * H * W + r * W + q, and runs of 4 k are 16 aligned bytes.
+template <int ROWS, int THREADS>
+struct PatchOperand {
+    using Map = KOctets<ROWS, THREADS>;
+    const GemmArgs::PatchB* v;
+    int64_t col0;
+    int64_t cols;
+    uint32_t col_off[Map::kPer];
+
+    __device__ __forceinline__ uint32_t ColOff(int64_t n) const {
+        // Columns past the operand read its last one.
+        const uint32_t nn = static_cast<uint32_t>(n < cols ? n : cols - 1);
+        uint32_t rem;
+        const uint32_t img = DivMod(v->div_plane, nn, rem);
+        uint32_t ow;
+        const uint32_t oh = DivMod(v->div_ow, rem, ow);
+        return (img * static_cast<uint32_t>(v->c) * static_cast<uint32_t>(v->in_h) +
+                oh * static_cast<uint32_t>(v->kh)) *
+                   static_cast<uint32_t>(v->in_w) +
+               ow * static_cast<uint32_t>(v->kw);
+    }
+    __device__ __forceinline__ void Init(const GemmArgs::PatchB& pv, int64_t first, int64_t total) {
+        v = &pv;
+        col0 = first;
+        cols = total;
+#pragma unroll
+        for (int p = 0; p < Map::kPer; ++p) {
+            col_off[p] = ColOff(first + Map::Row(static_cast<int>(threadIdx.x) + p * THREADS));
         }
     }
     __device__ __forceinline__ uint32_t KOff(uint32_t k) const {
@@ -90,32 +172,53 @@ struct PatchLoader {
         const uint32_t r = DivMod(v->div_kw, rem, q);
         return (c * static_cast<uint32_t>(v->in_h) + r) * static_cast<uint32_t>(v->in_w) + q;
     }
-    __device__ __forceinline__ void load(int64_t k0, Stage& s) const {
-        const int tid = threadIdx.x;
+    __device__ __forceinline__ void LoadFull(int p, int64_t k0, nert_floatx4& lo, nert_floatx4& hi) const {
+        const int q = static_cast<int>(threadIdx.x) + p * THREADS;
+        const uint32_t k = static_cast<uint32_t>(k0) + static_cast<uint32_t>(8 * Map::Oct(q));
+        lo = *reinterpret_cast<const nert_floatx4*>(v->x + col_off[p] + KOff(k));
+        hi = *reinterpret_cast<const nert_floatx4*>(v->x + col_off[p] + KOff(k + 4));
+    }
+    __device__ __forceinline__ float At(int row, int64_t k) const {
+        return v->x[ColOff(col0 + row) + KOff(static_cast<uint32_t>(k))];
+    }
+};
+
+// One thread's octets of a K step in registers.
+template <class Operand, int ROWS, int THREADS>
+struct OctetStage {
+    using Map = typename Operand::Map;
+    nert_floatx4 lo[Map::kPer];
+    nert_floatx4 hi[Map::kPer];
+
+    __device__ __forceinline__ void LoadFull(int p, const Operand& op, int64_t k0) { op.LoadFull(p, k0, lo[p], hi[p]); }
+    __device__ __forceinline__ void LoadFull(const Operand& op, int64_t k0) {
 #pragma unroll
-        for (int p = 0; p < kPer; ++p) {
-            const int q = tid + p * THREADS;
-            const uint32_t k = static_cast<uint32_t>(k0) + static_cast<uint32_t>((q % (BK / 4)) * 4);
-            if constexpr (!CHECKED) {
-                if (kQuads % THREADS != 0 && q >= kQuads) {
-                    continue; // this thread owns no quad in this pass
-                }
-                const nert_floatx4 val = *reinterpret_cast<const nert_floatx4*>(v->x + col_off[p] + KOff(k));
-                s.v[p][0] = val[0];
-                s.v[p][1] = val[1];
-                s.v[p][2] = val[2];
-                s.v[p][3] = val[3];
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const bool ok = col_ok[p] && k + e < k_total;
-                    const float x = v->x[ok ? col_off[p] + KOff(k + e) : 0];
-                    s.v[p][e] = ok ? x : 0.f;
-                }
-            }
+        for (int p = 0; p < Map::kPer; ++p) {
+            LoadFull(p, op, k0);
         }
     }
-    __device__ __forceinline__ void store(const Stage& s, float* lds) const { Rows{}.store(s, lds); }
+    // The rest of K, less than a step: clamped addresses, zero past k_end.
+    __device__ __forceinline__ void LoadTail(const Operand& op, int64_t k0, int64_t k_end) {
+#pragma unroll
+        for (int p = 0; p < Map::kPer; ++p) {
+            const int q = static_cast<int>(threadIdx.x) + p * THREADS;
+            const int64_t k = k0 + 8 * Map::Oct(q);
+            auto at = [&](int e) {
+                const float f = op.At(Map::Row(q), k + e < k_end ? k + e : k_end - 1);
+                return k + e < k_end ? f : 0.0f;
+            };
+            lo[p] = nert_floatx4{at(0), at(1), at(2), at(3)};
+            hi[p] = nert_floatx4{at(4), at(5), at(6), at(7)};
+        }
+    }
+    __device__ __forceinline__ void Store(int p, uint32_t* lds) const {
+        const int slot = Map::Slot(static_cast<int>(threadIdx.x) + p * THREADS);
+        const SplitOctet o = Split8(lo[p], hi[p]);
+#pragma unroll
+        for (int piece = 0; piece < 3; ++piece) {
+            *reinterpret_cast<nert_uintx4*>(lds + piece * ROWS * 16 + slot * 4) = o.piece[piece];
+        }
+    }
 };
 
 // The epilogue of every GEMM kernel: alpha * acc, plus beta * bias, then the
@@ -140,65 +243,89 @@ __device__ __forceinline__ float FinishGemm(const GemmArgs& p, float acc, int64_
     return FinishWith(p, acc, p.has_bias ? p.bias[r * p.bias_sm + c * p.bias_sn] : 0.0f);
 }
 
-// Writes a workgroup's accumulators: raw partial sums (finish = false) or
-// finished outputs. Per 32x32 block, every bias load comes from a clamped,
-// always-valid address and all sixteen addresses are formed before the first
-// store, so the loads and stores of a lane are in flight together instead
-// of one guarded access and one wait after another.
-template <class Shape>
-__device__ __forceinline__ void GemmEpilogue(const GemmArgs& p, const Accum<Shape>& acc, float* out, int64_t row0,
-                                             int64_t col0, bool finish) {
+// Writes a wave's sums: raw partial sums (finish = false) or finished outputs.
+// A lane holds four consecutive columns of one row per block, stored as 16
+// bytes when the row pitch and the output allow.
+template <class Tile>
+__device__ __forceinline__ void GemmEpilogue(const GemmArgs& p, const SplitAccum<Tile::kRB, Tile::kCB>& acc,
+                                             float* out, int64_t row0, int64_t col0, bool finish) {
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int wave_m = wave % Shape::kWavesM;
-    const int wave_n = wave / Shape::kWavesM;
-    const int half = lane >> 5;
     // Finished outputs follow the output layout (GemmOutIndex); raw partial
     // sums stay dense [m][n].
     const bool grouped = finish && p.y_group > 0;
     const int64_t row_stride = grouped ? p.y_group : p.n;
+    const bool vec = row_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    const bool bias_vec = finish && p.has_bias && p.bias_sn == 1 && p.bias_sm % 4 == 0 && vec &&
+                          (reinterpret_cast<uintptr_t>(p.bias) & 15) == 0;
 #pragma unroll
-    for (int j = 0; j < Shape::kSubN; ++j) {
-        const int64_t gc = col0 + wave_n * Shape::kWaveN + 32 * j + (lane & 31);
-        const bool col_ok = gc < p.n;
-        const int64_t cc = col_ok ? gc : 0;
-        const int64_t col_base = grouped ? GemmOutIndex(p, 0, cc) : cc;
+    for (int j = 0; j < Tile::kCB; ++j) {
+        const int64_t c = col0 + 16 * j + 4 * (lane >> 4);
+        if (c >= p.n) {
+            continue;
+        }
+        const int64_t col_base = grouped ? GemmOutIndex(p, 0, c) : c;
+        const bool quad = vec && c + 4 <= p.n;
 #pragma unroll
-        for (int i = 0; i < Shape::kSubM; ++i) {
-            const int64_t r0 = row0 + wave_m * Shape::kWaveM + 32 * i + 4 * half;
-            float* base = out + r0 * row_stride + col_base;
-            float value[16];
-            bool ok[16];
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int64_t r = r0 + 8 * (v >> 2) + (v & 3);
-                ok[v] = col_ok && r < p.m;
-                float bias = 0.0f;
-                if (finish && p.has_bias) {
-                    const int64_t rr = r < p.m ? r : p.m - 1;
-                    bias = p.bias[rr * p.bias_sm + cc * p.bias_sn];
-                }
-                value[v] = finish ? FinishWith(p, acc.c[i][j][v], bias) : acc.c[i][j][v];
+        for (int i = 0; i < Tile::kRB; ++i) {
+            const int64_t r = row0 + 16 * i + (lane & 15);
+            if (r >= p.m) {
+                continue;
             }
+            float* at = out + r * row_stride + col_base;
+            nert_floatx4 value = acc.big[i][j];
+            if (finish) {
+                nert_floatx4 bias{0.0f, 0.0f, 0.0f, 0.0f};
+                if (bias_vec && quad) {
+                    bias = *reinterpret_cast<const nert_floatx4*>(p.bias + r * p.bias_sm + c);
+                } else if (p.has_bias) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                if (ok[v]) {
-                    base[(8 * (v >> 2) + (v & 3)) * row_stride] = value[v];
+                    for (int e = 0; e < 4; ++e) {
+                        const int64_t cc = c + e < p.n ? c + e : p.n - 1;
+                        bias[e] = p.bias[r * p.bias_sm + cc * p.bias_sn];
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    value[e] = FinishWith(p, value[e], bias[e]);
+                }
+            }
+            if (quad) {
+                *reinterpret_cast<nert_floatx4*>(at) = value;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (c + e < p.n) {
+                        at[e] = value[e];
+                    }
                 }
             }
         }
     }
 }
 
-template <class Shape, bool A_KCONTIG, bool B_NCONTIG, int FLUSH, bool B_PATCH = false>
-__global__ __launch_bounds__(Shape::kThreads) void GemmKernel(GemmArgs p) {
-    __shared__ __attribute__((aligned(16))) float lds[2 * (Shape::kLdsA + Shape::kLdsB)];
-    const int64_t tiles_m = (p.m + Shape::kBM - 1) / Shape::kBM;
-    const int64_t tile = blockIdx.x;
-    const int64_t tm = tile % tiles_m;
-    const int64_t tn = tile / tiles_m;
-    const int64_t row0 = tm * Shape::kBM;
-    const int64_t col0 = tn * Shape::kBN;
+// Tile of workgroup i of `count`: workgroups are dispatched round-robin over
+// the 8 XCDs, each with its own L2, so XCD i % 8 takes one contiguous run of
+// tiles, whose neighbours share operand rows or columns in that L2.
+__device__ __forceinline__ int64_t GemmTileOrder(int64_t i, int64_t count) {
+    const int64_t whole = count / 8 * 8;
+    return i < whole ? (i % 8) * (whole / 8) + i / 8 : i;
+}
+
+// Y tile = A tile * B tile on the bf16 matrix cores (split_mma.hpp). Per K
+// step of 32 the workgroup splits its BM + BN operand rows into LDS once
+// (global loads of the next step in flight under the MFMAs), then every wave
+// runs 6 kRB kCB MFMAs of 16 x 16 x 32 from it.
+template <class Tile, bool A_KCONTIG, bool B_NCONTIG, bool B_PATCH = false, class Offset = uint32_t>
+__global__ __launch_bounds__(Tile::kThreads, 2) void GemmKernel(GemmArgs p) {
+    constexpr int RB = Tile::kRB;
+    constexpr int CB = Tile::kCB;
+    constexpr int T = Tile::kThreads;
+    constexpr int kBuffer = kOperandLds<Tile::kBM> + kOperandLds<Tile::kBN>;
+    extern __shared__ __attribute__((aligned(16))) uint32_t lds[]; // two buffers
+    const int64_t tiles_m = (p.m + Tile::kBM - 1) / Tile::kBM;
+    const int64_t tile = GemmTileOrder(blockIdx.x, gridDim.x);
+    const int64_t row0 = (tile % tiles_m) * Tile::kBM;
+    const int64_t col0 = (tile / tiles_m) * Tile::kBN;
     const int64_t batch = blockIdx.y;
     const int split = blockIdx.z;
 
@@ -212,8 +339,6 @@ __global__ __launch_bounds__(Shape::kThreads) void GemmKernel(GemmArgs p) {
         a_off += idx * p.a_bs[d];
         b_off += idx * p.b_bs[d];
     }
-    const float* a = p.a + a_off;
-    const float* b = p.b + b_off;
 
     const int64_t k_begin = static_cast<int64_t>(split) * p.k_per_split;
     int64_t k_end = k_begin + p.k_per_split;
@@ -221,64 +346,143 @@ __global__ __launch_bounds__(Shape::kThreads) void GemmKernel(GemmArgs p) {
         k_end = p.k;
     }
 
-    Accum<Shape> acc;
-    acc.zero();
-    // Tiles with 16-byte aligned rows take unchecked float4 loads for every
-    // full K tile; the K remainder uses the checked form. So do edge tiles
-    // whose missing rows (or columns) the unchecked loaders can stand in for
-    // with valid ones -- any count along a K-contiguous operand, whole quads
-    // along a row-contiguous one: those rows only reach outputs that are never
-    // stored, and the stored outputs sum the same products in the same order.
-    const bool a_vec = (A_KCONTIG ? p.a_sm : p.a_sk) % 4 == 0 && ((reinterpret_cast<uintptr_t>(a) & 15) == 0);
-    const bool b_vec =
-        B_PATCH || ((B_NCONTIG ? p.b_sk : p.b_sn) % 4 == 0 && ((reinterpret_cast<uintptr_t>(b) & 15) == 0));
-    const bool a_rows = row0 + Shape::kBM <= p.m || A_KCONTIG || p.m % 4 == 0;
-    const bool b_cols = col0 + Shape::kBN <= p.n || !B_NCONTIG || p.n % 4 == 0;
-    const bool interior = a_vec && b_vec && a_rows && b_cols;
-    const int64_t k_full = interior ? k_begin + (k_end - k_begin) / Shape::kBK * Shape::kBK : k_begin;
-    if (k_full > k_begin) {
-        const auto aload = MakeOperand<Shape::kBM, Shape::kBK, Shape::kThreads, Shape::kPitchA, A_KCONTIG, false>(
-            a, row0, p.a_sm, p.a_sk, p.m, k_full);
-        if constexpr (B_PATCH) {
-            PatchLoader<Shape::kBN, Shape::kBK, Shape::kThreads, Shape::kPitchB, false> bload;
-            bload.init(p.patch, col0, p.n, k_full);
-            MainLoop<Shape, FLUSH>(aload, bload, k_begin, k_full, lds, acc);
-        } else {
-            const auto bload = MakeOperand<Shape::kBN, Shape::kBK, Shape::kThreads, Shape::kPitchB, !B_NCONTIG, false>(
-                b, col0, p.b_sn, p.b_sk, p.n, k_full);
-            MainLoop<Shape, FLUSH>(aload, bload, k_begin, k_full, lds, acc);
-        }
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int wave_row = (wave % Tile::kWavesM) * Tile::kRows;
+    const int wave_col = (wave / Tile::kWavesM) * Tile::kCols;
+
+    using OperandA = StridedOperand<Tile::kBM, T, A_KCONTIG, Offset>;
+    using OperandB = std::conditional_t<B_PATCH, PatchOperand<Tile::kBN, T>,
+                                        StridedOperand<Tile::kBN, T, !B_NCONTIG, Offset>>;
+    OperandA a;
+    OperandB b;
+    a.Init(p.a + a_off, row0, p.a_sm, p.a_sk, p.m);
+    if constexpr (B_PATCH) {
+        b.Init(p.patch, col0, p.n);
+    } else {
+        b.Init(p.b + b_off, col0, p.b_sn, p.b_sk, p.n);
     }
-    if (k_full < k_end) {
-        const auto aload = MakeOperand<Shape::kBM, Shape::kBK, Shape::kThreads, Shape::kPitchA, A_KCONTIG, true>(
-            a, row0, p.a_sm, p.a_sk, p.m, k_end);
-        if constexpr (B_PATCH) {
-            PatchLoader<Shape::kBN, Shape::kBK, Shape::kThreads, Shape::kPitchB, true> bload;
-            bload.init(p.patch, col0, p.n, k_end);
-            MainLoop<Shape, FLUSH>(aload, bload, k_full, k_end, lds, acc);
-        } else {
-            const auto bload = MakeOperand<Shape::kBN, Shape::kBK, Shape::kThreads, Shape::kPitchB, !B_NCONTIG, true>(
-                b, col0, p.b_sn, p.b_sk, p.n, k_end);
-            MainLoop<Shape, FLUSH>(aload, bload, k_full, k_end, lds, acc);
+
+    SplitAccum<RB, CB> acc;
+    acc.Zero();
+    OctetStage<OperandA, Tile::kBM, T> sa;
+    OctetStage<OperandB, Tile::kBN, T> sb;
+    // What K leaves over whole steps goes first, so that the loop loads
+    // whole steps only.
+    const int64_t rest = (k_end - k_begin) % 32;
+    const int64_t steps = (k_end - k_begin + 31) / 32;
+    const int64_t k_first = rest != 0 ? k_begin - 32 : k_begin; // of step 0, were it whole
+    const int64_t k_last = k_end - rest - 32;                   // the last whole step's, where a prefetch stops
+    if (rest != 0) {
+        sa.LoadTail(a, k_end - rest, k_end);
+        sb.LoadTail(b, k_end - rest, k_end);
+    } else if (steps > 0) {
+        sa.LoadFull(a, k_begin);
+        sb.LoadFull(b, k_begin);
+    }
+    // One step: multiplies the buffer at `use`. With STAGE the next step's
+    // octets, in registers since the step before, are meanwhile split into
+    // the buffer at `fill`, and K = `next` is loaded: each row block's MFMAs take a share of the octets, and the group barriers spread
+    // their vector instructions between the MFMAs, whose issue slots they fit.
+    const int frag_a = (wave_row / 16 * 64 + lane) * 4;
+    const int frag_b = kOperandLds<Tile::kBM> + (wave_col / 16 * 64 + lane) * 4;
+    auto step_body = [&](auto stage_tag, const uint32_t* use, uint32_t* fill, int64_t next) {
+        constexpr bool kStage = decltype(stage_tag)::value;
+        constexpr int kOctets = OperandA::Map::kPer + OperandB::Map::kPer;
+        nert_uintx4 col[CB][3];
+        nert_uintx4 row[2][3];
+#pragma unroll
+        for (int piece = 0; piece < 3; ++piece) {
+            row[0][piece] = *reinterpret_cast<const nert_uintx4*>(use + frag_a + piece * Tile::kBM * 16);
         }
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+#pragma unroll
+            for (int piece = 0; piece < 3; ++piece) {
+                col[j][piece] = *reinterpret_cast<const nert_uintx4*>(use + frag_b + piece * Tile::kBN * 16 + j * 256);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            if (i + 1 < RB) {
+#pragma unroll
+                for (int piece = 0; piece < 3; ++piece) {
+                    row[(i + 1) % 2][piece] = *reinterpret_cast<const nert_uintx4*>(
+                        use + frag_a + piece * Tile::kBM * 16 + (i + 1) * 256);
+                }
+            }
+            acc.Step(i, row[i % 2], col);
+            if constexpr (kStage) {
+                constexpr int kMfmas = 6 * CB;
+                int octets = 0;
+#pragma unroll
+                for (int o = 0; o < kOctets; ++o) {
+                    if (o * RB / kOctets != i) {
+                        continue;
+                    }
+                    ++octets;
+                    if (o < OperandA::Map::kPer) {
+                        sa.Store(o, fill);
+                        sa.LoadFull(o, a, next);
+                    } else {
+                        sb.Store(o - OperandA::Map::kPer, fill + kOperandLds<Tile::kBM>);
+                        sb.LoadFull(o - OperandA::Map::kPer, b, next);
+                    }
+                }
+                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0); // LDS reads
+#pragma unroll
+                for (int s = 0; s < kMfmas / 2; ++s) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0); // MFMA
+                    if (octets > 0) {
+                        __builtin_amdgcn_sched_group_barrier(0x002, 60 * kOctets / RB / (kMfmas / 2) + 1, 0); // VALU
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    if (steps > 0) {
+#pragma unroll
+        for (int o = 0; o < OperandA::Map::kPer; ++o) {
+            sa.Store(o, lds);
+        }
+#pragma unroll
+        for (int o = 0; o < OperandB::Map::kPer; ++o) {
+            sb.Store(o, lds + kOperandLds<Tile::kBM>);
+        }
+        if (steps > 1) {
+            sa.LoadFull(a, k_first + 32);
+            sb.LoadFull(b, k_first + 32);
+        }
+        __syncthreads();
+        uint32_t buffer = 0;
+        for (int64_t step = 0; step + 1 < steps; ++step) {
+            step_body(std::true_type{}, lds + buffer, lds + (kBuffer - buffer), min(k_first + 32 * (step + 2), k_last));
+            __syncthreads();
+            buffer = kBuffer - buffer;
+        }
+        step_body(std::false_type{}, lds + buffer, lds + buffer, k_last);
+    }
+    if (acc.Finish()) {
+        RerunFloat32(
+            acc, k_begin, k_end, [&](int i, int64_t k) { return a.At(wave_row + 16 * i + (lane & 15), k); },
+            [&](int j, int64_t k) { return b.At(wave_col + 16 * j + (lane & 15), k); });
     }
 
     const int64_t plane = p.m * p.n;
     if (p.counters != nullptr) {
         const int64_t t = batch * gridDim.x + tile;
-        float* slots = p.split_slots + t * gridDim.z * Shape::kBM * Shape::kBN;
-        if (FinishSplitTile<Shape, double>(acc, slots, p.counters + t, split, static_cast<int>(gridDim.z),
-                                           reinterpret_cast<int*>(lds))) {
-            GemmEpilogue<Shape>(p, acc, p.y + batch * plane, row0, col0, true);
+        float* slots = p.split_slots + t * gridDim.z * Tile::kBM * Tile::kBN;
+        if (FinishSplitParts<RB, CB, T, double>(acc, slots, p.counters + t, split, static_cast<int>(gridDim.z),
+                                                reinterpret_cast<int*>(lds))) {
+            GemmEpilogue<Tile>(p, acc, p.y + batch * plane, row0 + wave_row, col0 + wave_col, true);
         }
         return;
     }
-    if (p.partial != nullptr) {
-        GemmEpilogue<Shape>(p, acc, p.partial + (static_cast<int64_t>(split) * gridDim.y + batch) * plane, row0, col0,
-                            false);
-        return;
-    }
-    GemmEpilogue<Shape>(p, acc, p.y + batch * plane, row0, col0, true);
+    float* out = p.partial != nullptr ? p.partial + (static_cast<int64_t>(split) * gridDim.y + batch) * plane
+                                      : p.y + batch * plane;
+    GemmEpilogue<Tile>(p, acc, out, row0 + wave_row, col0 + wave_col, p.partial == nullptr);
 }
 
 // Sums the split-K partials in split order (deterministic), in double with
@@ -434,101 +638,107 @@ void LaunchSkinny(const GemmArgs& p, hipStream_t stream) {
     CheckLaunch("SkinnyGemmKernel launch");
 }
 
-// Tile shapes, chosen from a sweep over the BASELINE GEMM/MatMul shapes and
-// the ViT projections on MI355X: 8 waves of 64x32 for problems with at least
-// 1024 such tiles (4096^3: 135 TFLOP/s), 4 waves of 32x64 below that (more
-// workgroups in flight hide the load latency), 2 waves for M <= 32.
-constexpr int64_t kTwoLevelK = 1024;
-constexpr int64_t kChunkK = 512;
-using ShapeL = TileShape<128, 128, 16, 2, 4>; // 8 waves, 64x32 per wave
-using ShapeM = TileShape<64, 128, 16, 2, 2>;  // 4 waves, 32x64 per wave
-using ShapeS = TileShape<32, 64, 32, 1, 2>;   // 2 waves, skinny M
-// The M and L tiles with 32-deep K steps: half the LDS-store/barrier phases
-// per K, twice the LDS.
-using ShapeMK = TileShape<64, 128, 32, 2, 2>;  // 4 waves, 32x64 per wave
-using ShapeLK = TileShape<128, 128, 32, 2, 4>; // 8 waves, 64x32 per wave
-// 4 waves of 32x32 for products a few hundred 64x128 tiles cover unevenly
-// (N = 768 next to M ~ 3000: 294 such tiles on 256 CUs, 600 of these).
-using ShapeQ = TileShape<64, 64, 32, 2, 2>;
+// Tile shapes: 64 x 64 per wave where the problem has enough tiles for the
+// 512 workgroups the chip holds, smaller ones below.
+using TileL = GemmTile<128, 128, 2, 4>; // 64 x 32 per wave, 8 waves
+using TileM = GemmTile<64, 128, 2, 2>;  // 32 x 64 per wave
+using TileS = GemmTile<32, 64, 1, 2>;   // 32 x 32 per wave, few rows
+using TileN = GemmTile<128, 64, 2, 2>;  // 64 x 32 per wave
+using TileX = GemmTile<256, 128, 4, 2>; // 64 x 64 per wave, 8 waves
+using TileQ = GemmTile<64, 64, 2, 2>;   // 32 x 32 per wave
 
-template <class Shape>
+// Launches one instantiation with its two LDS buffers; beyond 64 KiB the
+// limit of a launch is raised once per process.
+template <class Tile, auto Kernel>
+void LaunchKernel(const GemmArgs& p, dim3 grid, hipStream_t stream) {
+    constexpr int kLds = 2 * 4 * (kOperandLds<Tile::kBM> + kOperandLds<Tile::kBN>);
+    if constexpr (kLds > 64 * 1024) {
+        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel),
+                                                             hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        Check(raised, "hipFuncSetAttribute(GemmKernel)");
+    }
+    Kernel<<<grid, Tile::kThreads, kLds, stream>>>(p);
+}
+
+template <class Tile, class Offset = uint32_t>
 void LaunchShape(GemmArgs p, int64_t batches, int splits, hipStream_t stream) {
-    const int64_t tiles = ((p.m + Shape::kBM - 1) / Shape::kBM) * ((p.n + Shape::kBN - 1) / Shape::kBN);
+    const int64_t tiles = ((p.m + Tile::kBM - 1) / Tile::kBM) * ((p.n + Tile::kBN - 1) / Tile::kBN);
     dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(batches), static_cast<unsigned>(splits));
     if (p.counters != nullptr) {
         p.split_slots = static_cast<float*>(
-            Workspace(tiles * batches * splits * Shape::kBM * Shape::kBN * static_cast<int64_t>(sizeof(float)), stream));
+            Workspace(tiles * batches * splits * Tile::kBM * Tile::kBN * static_cast<int64_t>(sizeof(float)), stream));
     }
-    dim3 block(Shape::kThreads);
     const bool a_k = p.a_sk == 1;
     const bool b_n = p.b_sn == 1;
-    // K ranges beyond kTwoLevelK accumulate in chunks of kChunkK (see
-    // MainLoop); shorter ones keep one set of accumulators (the second set
-    // costs occupancy).
-    const bool two_level = p.k_per_split > kTwoLevelK;
-    constexpr int kFlush = kChunkK / Shape::kBK;
     if (p.patch.x != nullptr) {
         // (A K-contiguous, one batch: LaunchGemm checks.)
-        two_level ? GemmKernel<Shape, true, false, kFlush, true><<<grid, block, 0, stream>>>(p)
-                  : GemmKernel<Shape, true, false, 0, true><<<grid, block, 0, stream>>>(p);
+        LaunchKernel<Tile, GemmKernel<Tile, true, false, true, Offset>>(p, grid, stream);
     } else if (a_k && b_n) {
-        two_level ? GemmKernel<Shape, true, true, kFlush><<<grid, block, 0, stream>>>(p)
-                  : GemmKernel<Shape, true, true, 0><<<grid, block, 0, stream>>>(p);
+        LaunchKernel<Tile, GemmKernel<Tile, true, true, false, Offset>>(p, grid, stream);
     } else if (a_k) {
-        two_level ? GemmKernel<Shape, true, false, kFlush><<<grid, block, 0, stream>>>(p)
-                  : GemmKernel<Shape, true, false, 0><<<grid, block, 0, stream>>>(p);
+        LaunchKernel<Tile, GemmKernel<Tile, true, false, false, Offset>>(p, grid, stream);
     } else if (b_n) {
-        two_level ? GemmKernel<Shape, false, true, kFlush><<<grid, block, 0, stream>>>(p)
-                  : GemmKernel<Shape, false, true, 0><<<grid, block, 0, stream>>>(p);
+        LaunchKernel<Tile, GemmKernel<Tile, false, true, false, Offset>>(p, grid, stream);
     } else {
-        two_level ? GemmKernel<Shape, false, false, kFlush><<<grid, block, 0, stream>>>(p)
-                  : GemmKernel<Shape, false, false, 0><<<grid, block, 0, stream>>>(p);
+        LaunchKernel<Tile, GemmKernel<Tile, false, false, false, Offset>>(p, grid, stream);
     }
     CheckLaunch("GemmKernel launch");
 }
 
-template <class Shape>
+template <class Tile>
 int64_t TileCount(const GemmArgs& p, int64_t batches) {
-    return ((p.m + Shape::kBM - 1) / Shape::kBM) * ((p.n + Shape::kBN - 1) / Shape::kBN) * batches;
+    return ((p.m + Tile::kBM - 1) / Tile::kBM) * ((p.n + Tile::kBN - 1) / Tile::kBN) * batches;
 }
 
 } // namespace
 
 namespace {
 
-// One configuration: tile shape (0 L, 1 M, 2 S, 3 MK, 4 LK, 5 Q) and split-K count
+// Strides that 32-bit offsets reach in the largest tile.
+bool NarrowOperands(const GemmArgs& p) {
+    using KSide = StridedOperand<TileX::kBM, TileX::kThreads, true, uint32_t>;
+    using RowSide = StridedOperand<TileX::kBM, TileX::kThreads, false, uint32_t>;
+    const bool a = p.a_sk == 1 ? KSide::Narrow(p.a_sm, 1) : RowSide::Narrow(1, p.a_sk);
+    const bool b = p.patch.x != nullptr || (p.b_sn == 1 ? RowSide::Narrow(1, p.b_sk) : KSide::Narrow(p.b_sn, 1));
+    return a && b;
+}
+
+// One configuration: tile shape (0 L, 1 M, 2 S, 3 N, 4 X, 5 Q) and split-K count
 // (0: the PlanSplits choice for that shape).
 void LaunchConfig(GemmArgs p, int64_t batches, int shape, int force_splits, hipStream_t stream) {
+    const bool narrow = NarrowOperands(p);
+    if (!narrow) {
+        shape = 5;
+    }
     int64_t tiles;
-    int64_t min_k_tiles = 8;
-    int bk = ShapeL::kBK;
-    if (shape == 0) {
-        tiles = TileCount<ShapeL>(p, batches);
-    } else if (shape == 1) {
-        tiles = TileCount<ShapeM>(p, batches);
-    } else if (shape == 3) {
-        tiles = TileCount<ShapeMK>(p, batches);
-        min_k_tiles = 4;
-        bk = ShapeMK::kBK;
-    } else if (shape == 4) {
-        tiles = TileCount<ShapeLK>(p, batches);
-        min_k_tiles = 4;
-        bk = ShapeLK::kBK;
-    } else if (shape == 5) {
-        tiles = TileCount<ShapeQ>(p, batches);
-        min_k_tiles = 4;
-        bk = ShapeQ::kBK;
-    } else {
-        tiles = TileCount<ShapeS>(p, batches);
-        min_k_tiles = 2;
-        bk = ShapeS::kBK;
+    int64_t resident = 2 * kResidentBlocks;
+    constexpr int bk = TileL::kBK;
+    switch (shape) {
+    case 0:
+        tiles = TileCount<TileL>(p, batches);
+        resident = kResidentBlocks / 2;
+        break;
+    case 1:
+        tiles = TileCount<TileM>(p, batches);
+        break;
+    case 3:
+        tiles = TileCount<TileN>(p, batches);
+        break;
+    case 4:
+        tiles = TileCount<TileX>(p, batches);
+        resident = kResidentBlocks / 2;
+        break;
+    case 5:
+        tiles = TileCount<TileQ>(p, batches);
+        break;
+    default:
+        tiles = TileCount<TileS>(p, batches);
+        break;
     }
     const int64_t k_tiles = (p.k + bk - 1) / bk;
-    // The 2- and 4-wave shapes keep about 1024 workgroups resident.
-    const bool eight_waves = shape == 0 || shape == 4;
     int splits = force_splits > 0
                      ? static_cast<int>(std::min<int64_t>(force_splits, std::max<int64_t>(k_tiles, 1)))
-                     : PlanSplits(tiles, k_tiles, eight_waves ? kResidentBlocks : 2 * kResidentBlocks, min_k_tiles, 32);
+                     : PlanSplits(tiles, k_tiles, resident, 4, 32);
     p.k_per_split = ((k_tiles + splits - 1) / splits) * bk;
     if (p.k == 0) {
         p.k_per_split = 0;
@@ -548,22 +758,23 @@ void LaunchConfig(GemmArgs p, int64_t batches, int shape, int force_splits, hipS
     }
     switch (shape) {
     case 0:
-        LaunchShape<ShapeL>(p, batches, splits, stream);
+        LaunchShape<TileL>(p, batches, splits, stream);
         break;
     case 1:
-        LaunchShape<ShapeM>(p, batches, splits, stream);
+        LaunchShape<TileM>(p, batches, splits, stream);
         break;
     case 3:
-        LaunchShape<ShapeMK>(p, batches, splits, stream);
+        LaunchShape<TileN>(p, batches, splits, stream);
         break;
     case 4:
-        LaunchShape<ShapeLK>(p, batches, splits, stream);
+        LaunchShape<TileX>(p, batches, splits, stream);
         break;
     case 5:
-        LaunchShape<ShapeQ>(p, batches, splits, stream);
+        narrow ? LaunchShape<TileQ>(p, batches, splits, stream)
+               : LaunchShape<TileQ, int64_t>(p, batches, splits, stream);
         break;
     default:
-        LaunchShape<ShapeS>(p, batches, splits, stream);
+        LaunchShape<TileS>(p, batches, splits, stream);
         break;
     }
     if (splits > 1 && p.counters == nullptr) {
@@ -582,10 +793,8 @@ void LaunchConfig(GemmArgs p, int64_t batches, int shape, int force_splits, hipS
 }
 
 // Candidates: 0-11 shape i / 4 (L, M, S) with split count {PlanSplits, 1,
-// 2, 4}[i % 4]; 12 the skinny kernel; 13-24 shape 3 + (i - 13) / 4 (MK, LK,
+// 2, 4}[i % 4]; 12 the skinny kernel; 13-24 shape 3 + (i - 13) / 4 (N, X,
 // Q) with split count {...}[(i - 13) % 4].
-// Fallback (capture, tuning off): 8-wave 128x128 tiles for problems with at
-// least 1024 of them, 4-wave 64x128 below, 2-wave 32x64 for M <= 32.
 using GemmKey = std::array<int64_t, 10>;
 constexpr int kGemmSplits[4] = {0, 1, 2, 4};
 constexpr int kGemmCandidates = 25;
@@ -617,7 +826,10 @@ void LaunchGemm(GemmArgs p, int64_t batches, hipStream_t stream) {
                                  (reinterpret_cast<uintptr_t>(p.patch.x) & 15) != 0)) {
         throw Error("gemm: an in-place patch operand needs one batch, A K-contiguous and 16-byte runs");
     }
-    const int fallback_shape = p.m <= 32 ? 2 : (TileCount<ShapeL>(p, batches) < 1024 ? 1 : 0);
+    // Tuning off or under capture: the largest tile that still fills most of
+    // the chip (256 x 128 on 192 or more of the 256 CUs), few rows the 32-row
+    // tile, else 64 x 64.
+    const int fallback = TileCount<TileX>(p, batches) >= 192 ? 17 : p.m <= 32 ? 8 : 21;
     static std::mutex mu;
     static std::map<GemmKey, int> chosen;
     // The key leaves the epilogue out: a fused and an unfused call of the
@@ -638,7 +850,7 @@ void LaunchGemm(GemmArgs p, int64_t batches, hipStream_t stream) {
             return;
         }
     }
-    const int c = ChooseConfig("gemm", chosen, mu, key, y_bytes, stream, kGemmCandidates, 4 * fallback_shape,
+    const int c = ChooseConfig("gemm3", chosen, mu, key, y_bytes, stream, kGemmCandidates, fallback,
                                [&](int i, float* scratch) {
                                    GemmArgs q = p;
                                    q.y = scratch;
@@ -658,7 +870,7 @@ void LaunchGemm(GemmArgs p, int64_t batches, hipStream_t stream) {
     }
     // (A cached skinny choice with operands that lost its alignment takes
     // the fallback tiles.)
-    LaunchTiled(p, batches, c == kSkinnyCandidate ? 4 * fallback_shape : c, stream);
+    LaunchTiled(p, batches, c == kSkinnyCandidate ? fallback : c, stream);
 }
 
 } // namespace nert_hip

@@ -1,0 +1,270 @@
+#pragma once
+// float32 products on the bf16 matrix cores, with all 24 bits of both operands.
+//
+// A float32 is the exact sum of three bf16 numbers, x = h + m + l: h is x
+// rounded to bf16 (8 significant bits), m the rest rounded to bf16, l what is
+// left, which 8 bits hold. A product is then hh + (hm + mh) + (hl + mm + lh)
+// + (ml + lm + ll); the three products of the last bracket are below 2^-26 of
+// the whole, under a quarter of a float32 rounding, and are left out. The six
+// others run as v_mfma_f32_16x16x32_bf16, whose products are exact and whose
+// accumulators are float32: hh in one set of accumulators, the five small
+// ones in a second, added once at the end, so the small ones do not lose
+// their low bits against a large running sum.
+//
+// Why: on an MI355X the bf16 instruction sustains 2445 TFLOP/s (a loop of
+// nothing else), 407 TFLOP/s of such six-fold products, against 153 TFLOP/s
+// of v_mfma_f32_32x32x2_f32. Error against float64 for normal operands, 2-norm
+// relative, this form / the float32 instruction: K = 64 4.9e-8 / 1.4e-7,
+// K = 576 1.4e-7 / 4.3e-7, K = 1024 1.8e-7 / 5.6e-7, K = 4096 4.1e-7 / 1.1e-6;
+// with everything in one set of accumulators 1.1e-7, 3.6e-7, 4.8e-7, 1.0e-6,
+// and a bias towards minus infinity. (The instruction adds 32 products before
+// it rounds into the accumulator, the float32 one two.)
+//
+// Range: the matrix cores read subnormal bf16 numbers as zero, so operands
+// are scaled by 2^24 on the way in (exact) and results by 2^-48 on the way
+// out: then every piece of every float32, the subnormal ones included, is a
+// normal bf16 number or zero. What overflows instead (|x| >= 2^104, a sum
+// >= 2^80, infinities, NaN) leaves a non-finite accumulator; a wave that
+// finds one computes its whole block again with the float32 instruction
+// (kernels call their own loop for that), so such inputs give what plain
+// float32 arithmetic gives.
+//
+// v_mfma_f32_16x16x32_bf16 lane layout (wave64):
+//   A fragment: lane l holds A[row = l % 16][k = 8 * (l / 16) + 0..7]
+//   B fragment: lane l holds B[k = 8 * (l / 16) + 0..7][col = l % 16]
+//   D (4 regs): lane l, reg v holds D[row = 4 * (l / 16) + v][col = l % 16]
+// v_mfma_f32_16x16x4_f32: A[row = l % 16][k = l / 16], the same D.
+
+#include "common.hpp"
+
+namespace nert_hip {
+
+typedef __bf16 nert_bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 nert_bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr float kSplitScale = 16777216.0f;                   // 2^24, applied to each operand
+constexpr float kSplitUnscale = 1.0f / (16777216.0f * 16777216.0f); // 2^-48, applied to the sums
+
+// Eight consecutive k of one operand row, as a fragment's 16 bytes per piece.
+struct SplitOctet {
+    nert_uintx4 piece[3]; // h, m, l
+};
+
+__device__ __forceinline__ uint32_t PackBf16(float a, float b) {
+    const nert_floatx2 v{a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, nert_bf16x2)); // v_cvt_pk_bf16_f32
+}
+
+__device__ __forceinline__ float LowBf16(uint32_t pair) { return __builtin_bit_cast(float, pair << 16); }
+__device__ __forceinline__ float HighBf16(uint32_t pair) { return __builtin_bit_cast(float, pair & 0xffff0000u); }
+
+// The split of two floats (already scaled): 9 vector instructions.
+__device__ __forceinline__ void SplitPair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = PackBf16(a, b);
+    const float ra = a - LowBf16(h);
+    const float rb = b - HighBf16(h);
+    m = PackBf16(ra, rb);
+    l = PackBf16(ra - LowBf16(m), rb - HighBf16(m));
+}
+
+__device__ __forceinline__ SplitOctet Split8(nert_floatx4 lo, nert_floatx4 hi) {
+    uint32_t h[4], m[4], l[4];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        SplitPair(lo[2 * e] * kSplitScale, lo[2 * e + 1] * kSplitScale, h[e], m[e], l[e]);
+        SplitPair(hi[2 * e] * kSplitScale, hi[2 * e + 1] * kSplitScale, h[2 + e], m[2 + e], l[2 + e]);
+    }
+    return SplitOctet{{nert_uintx4{h[0], h[1], h[2], h[3]}, nert_uintx4{m[0], m[1], m[2], m[3]},
+                       nert_uintx4{l[0], l[1], l[2], l[3]}}};
+}
+
+__device__ __forceinline__ nert_floatx4 MfmaBf16(nert_uintx4 a, nert_uintx4 b, nert_floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(nert_bf16x8, a),
+                                                   __builtin_bit_cast(nert_bf16x8, b), c, 0, 0, 0);
+}
+
+// Accumulators of one wave: RB x CB blocks of 16 x 16, held transposed (the
+// column operand is the instruction's A): lane l, register v of block (i, j)
+// is output row 16 i + l % 16, column 16 j + 4 * (l / 16) + v, so a lane's
+// four registers are consecutive columns.
+template <int RB, int CB>
+struct SplitAccum {
+    nert_floatx4 big[RB][CB];   // hh, later the finished sums
+    nert_floatx4 small[RB][CB]; // the five other products
+
+    __device__ __forceinline__ void Zero() {
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+                big[i][j] = nert_floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                small[i][j] = nert_floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+    }
+
+    // One K = 32 step of row block i: `row` its fragment pieces, `col` those
+    // of every column block. The six products go round the column blocks, so
+    // MFMAs on one accumulator are CB apart; the smallest products first.
+    __device__ __forceinline__ void Step(int i, const nert_uintx4 (&row)[3], const nert_uintx4 (&col)[CB][3]) {
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            small[i][j] = MfmaBf16(col[j][1], row[1], small[i][j]);
+        }
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            small[i][j] = MfmaBf16(col[j][2], row[0], small[i][j]);
+        }
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            small[i][j] = MfmaBf16(col[j][0], row[2], small[i][j]);
+        }
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            small[i][j] = MfmaBf16(col[j][1], row[0], small[i][j]);
+        }
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            small[i][j] = MfmaBf16(col[j][0], row[1], small[i][j]);
+        }
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            big[i][j] = MfmaBf16(col[j][0], row[0], big[i][j]);
+        }
+    }
+
+    // Adds the two sets and undoes the scaling, in `big`; true (to the whole
+    // wave) when some sum is not finite and the block has to be computed
+    // again in float32.
+    __device__ __forceinline__ bool Finish() {
+        float bad = 0.0f;
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float s = big[i][j][v] + small[i][j][v];
+                    bad = fmaf(s, 0.0f, bad); // NaN as soon as one s is not finite
+                    big[i][j][v] = s * kSplitUnscale;
+                }
+            }
+        }
+        return __any(bad != 0.0f);
+    }
+};
+
+// The same block in float32, `row(i, k)` and `col(j, k)` giving this lane's
+// operand of row or column block i / j at k (zero outside the problem): k
+// runs over [k_begin, k_end) in chunks of 512, each summed by itself, into
+// acc.big. Reached for non-finite or huge values only.
+template <int RB, int CB, class Row, class Col>
+__device__ __forceinline__ void RerunFloat32(SplitAccum<RB, CB>& acc, int64_t k_begin, int64_t k_end, const Row& row, const Col& col) {
+    const int64_t lane_k = (threadIdx.x & 63) >> 4;
+    acc.Zero();
+#pragma unroll 1
+    for (int64_t k0 = k_begin; k0 < k_end; k0 += 512) {
+        const int64_t end = k0 + 512 < k_end ? k0 + 512 : k_end;
+        for (int64_t k = k0; k < end; k += 4) {
+            float r[RB];
+            float c[CB];
+#pragma unroll
+            for (int i = 0; i < RB; ++i) {
+                r[i] = k + lane_k < end ? row(i, k + lane_k) : 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+                c[j] = k + lane_k < end ? col(j, k + lane_k) : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < RB; ++i) {
+#pragma unroll
+                for (int j = 0; j < CB; ++j) {
+                    acc.small[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(c[j], r[i], acc.small[i][j], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+                acc.big[i][j] += acc.small[i][j];
+                acc.small[i][j] = nert_floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+    }
+}
+
+// Split tiles finished inside the kernel: every workgroup that computes one
+// part of a tile's K sum stores its sums to slot `part` of the tile's slots
+// (16-byte pieces in register order, consecutive threads at consecutive
+// addresses) and counts itself in the tile's counter; the one that completes
+// the count resets it, adds the parts in part order in type Sum, rounds once
+// and returns true to run the epilogue. See FinishSplitTile in mfma_tile.hpp
+// for the cache policy and the ordering; this is the same protocol for
+// another accumulator layout.
+template <int RB, int CB, int THREADS, class Sum>
+__device__ __forceinline__ bool FinishSplitParts(SplitAccum<RB, CB>& acc, float* slots, uint32_t* counter, int part,
+                                                 int parts, int* flag) {
+    constexpr int kDeviceCoherent = 16; // cache policy: sc1
+    constexpr int kSlot = RB * CB * THREADS * 16; // bytes
+    const __amdgpu_buffer_rsrc_t r =
+        __builtin_amdgcn_make_buffer_rsrc(slots, static_cast<short>(0), parts * kSlot, 0x00020000);
+    const int at = static_cast<int>(threadIdx.x) * 16;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nert_uintx4, acc.big[i][j]), r,
+                                                   part * kSlot + (i * CB + j) * THREADS * 16 + at, 0,
+                                                   kDeviceCoherent);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool last = before + 1 == static_cast<uint32_t>(parts);
+        if (last) {
+            __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        *flag = last ? 1 : 0;
+    }
+    __syncthreads();
+    if (*flag == 0) {
+        return false;
+    }
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            Sum sum[4];
+            for (int q0 = 0; q0 < parts; q0 += 4) { // four parts' loads in flight
+                nert_floatx4 x[4];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    const int q = min(q0 + d, parts - 1);
+                    x[d] = __builtin_bit_cast(
+                        nert_floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                                          r, q * kSlot + (i * CB + j) * THREADS * 16 + at, 0, kDeviceCoherent));
+                }
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    if (q0 + d < parts) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            sum[e] = q0 + d == 0 ? static_cast<Sum>(x[d][e]) : sum[e] + static_cast<Sum>(x[d][e]);
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc.big[i][j][e] = static_cast<float>(sum[e]);
+            }
+        }
+    }
+    return true;
+}
+
+} // namespace nert_hip

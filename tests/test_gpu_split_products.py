@@ -1,0 +1,78 @@
+"""The products on the bf16 matrix cores (nert_amd/csrc/split_mma.hpp) against
+float64: edge sizes, both transposes, and the values whose split needs care
+(subnormal, huge, infinite and NaN operands)."""
+
+import numpy as np
+import pytest
+
+from nert_amd.device import DeviceArray, run_node
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+def _gemm(a, b, ta=0, tb=0, c=None):
+    m, n = (a.shape[1] if ta else a.shape[0]), (b.shape[0] if tb else b.shape[1])
+    y = DeviceArray((m, n), F)
+    ins = [DeviceArray.from_host(v) for v in ([a, b] if c is None else [a, b, c])]
+    run_node("Gemm", ins, [y], {"transA": ta, "transB": tb})
+    return y.to_host()
+
+
+def _bound(a, b, k):
+    """Every K step of 32 rounds each of two accumulators once, at most half
+    an ulp (2^-24) of the sum of the products' sizes; the left-out products
+    are below 2^-25 of it, the last additions add three roundings."""
+    return (2 * (k / 32 + 2) + 4) * 2.0 ** -24 * (np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64)))
+
+
+# Edges of the 32 .. 256 row tiles, of K's steps of 32, and of split K.
+SIZES = [(33, 1, 1), (64, 64, 31), (65, 63, 33), (128, 129, 32), (129, 255, 65), (257, 130, 96), (40, 48, 1100),
+         (300, 500, 161), (513, 384, 2048)]
+
+
+@pytest.mark.parametrize("m,n,k", SIZES)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_split_gemm_edges(gpu, m, n, k, ta, tb):
+    rng = np.random.default_rng(m * n + k)
+    a, b = rng.standard_normal((m, k)).astype(F), rng.standard_normal((k, n)).astype(F)
+    y = _gemm(np.ascontiguousarray(a.T) if ta else a, np.ascontiguousarray(b.T) if tb else b, ta, tb)
+    err = np.abs(y - a.astype(np.float64) @ b.astype(np.float64))
+    assert np.all(err <= _bound(a, b, k)), float((err / _bound(a, b, k)).max())
+
+
+@pytest.mark.parametrize("candidate", [0, 4, 8, 13, 17, 21, 24])
+def test_split_gemm_special_values(gpu, monkeypatch, candidate):
+    """Infinities and NaN land where float32 arithmetic puts them, sums past
+    2^80 keep their value, and subnormal operands keep all their bits."""
+    monkeypatch.setenv("NERT_HIP_GEMM_CANDIDATE", str(candidate))
+    rng = np.random.default_rng(7)
+    m, n, k = 140, 150, 200
+    a, b = rng.standard_normal((m, k)).astype(F), rng.standard_normal((k, n)).astype(F)
+    a[3, 5], a[70, 9], a[71, 0] = np.inf, -np.inf, np.nan
+    a[100] *= F(1e34)
+    a[120] = rng.standard_normal(k).astype(F) * F(1e-41)
+    a[121] = F(3e38)
+    b[:, 4] = rng.standard_normal(k).astype(F) * F(1e-3)
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+    y = _gemm(a, b)
+    for r in (3, 70, 71):
+        np.testing.assert_array_equal(np.isnan(y[r]), np.isnan(want[r]))
+        inf = np.isinf(want[r])
+        np.testing.assert_array_equal(y[r][inf], want[r][inf])
+    plain = [r for r in range(m) if r not in (3, 70, 71, 121)]
+    # (Results near the smallest subnormal, 2^-149, round to a multiple of it.)
+    bound = 2 * _bound(a[plain], b, k) + 2.0 ** -149 * (k / 32 + 2)
+    assert np.all(np.abs(y[plain] - want[plain]) <= bound)
+    big = np.abs(want[121]) < 3e38  # partial sums may pass the largest float32 on the way
+    same = np.isfinite(y[121]) & big
+    np.testing.assert_allclose(y[121][same], want[121][same], rtol=1e-4, atol=1e34)
+
+
+def test_split_gemm_exact_integers(gpu):
+    """Whole numbers whose products and sums fit 24 bits come out exact."""
+    rng = np.random.default_rng(3)
+    a = rng.integers(-500, 500, (200, 60)).astype(F)
+    b = rng.integers(-500, 500, (60, 170)).astype(F)
+    np.testing.assert_array_equal(_gemm(a, b), (a.astype(np.float64) @ b.astype(np.float64)).astype(F))
