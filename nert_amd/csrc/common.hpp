@@ -39,6 +39,8 @@ inline hipStream_t StreamOr(void* stream) {
 // slot 0 for its partials) holds it in slot 1.
 constexpr int kWorkspaceSlots = 2;
 void* Workspace(int64_t bytes, hipStream_t stream, int slot = 0);
+// Whether a slot already holds that many bytes, so that it would not grow.
+bool WorkspaceHolds(int64_t bytes, int slot);
 
 // A 64-byte device flag block (zeroed at creation) used by rows that must
 // report data-dependent errors (out-of-range indices, integer division by

@@ -27,70 +27,13 @@
 #include <mutex>
 #include <type_traits>
 
+#include "conv_args.hpp"
 #include "gemm_engine.hpp"
-#include "tune.hpp"
 #include "mfma_tile.hpp"
 #include "../../include/nert_hip.h"
 
 namespace nert_hip {
 namespace {
-
-struct ConvArgs {
-    const float* x;
-    const float* w;
-    // W again in the order the 3x3 LDS-patch kernel stores it, or null: per
-    // output channel, blocks of 8 input channels, in a block the taps, in a
-    // tap the 8 channels ([M][C_g / 8][KH * KW][8]); that kernel then copies
-    // it to LDS with 16-byte stores instead of transposing 4-byte ones.
-    // Every other kernel reads `w`.
-    const float* w_packed;
-    const float* bias;
-    float* y;
-    int64_t batch, c, m, group;
-    int64_t cg, mg, kg; // channels per group, outputs per group, K per group
-    int32_t in_d, in_h, in_w;
-    int32_t k_d, k_h, k_w;
-    int32_t out_d, out_h, out_w;
-    int32_t s_d, s_h, s_w;
-    int32_t d_d, d_h, d_w;
-    int32_t p_d, p_h, p_w;
-    int64_t plane_out; // OD*OH*OW
-    int64_t plane_in;  // ID*IH*IW
-    int64_t n_total;   // batch * plane_out
-    FastDiv div_kvol, div_khw, div_kw;
-    int64_t k_per_split;
-    float* partial; // [splits][group][M_g][N] when split
-    // Optional epilogue (fused rows): y = act(acc + bias + residual), in that
-    // order, so the result equals Conv, then Add, then the activation rows
-    // bit for bit.
-    const float* residual; // same layout as y, or null
-    int32_t act;           // 0 none, 1 Relu, 2 SiLU (x * Sigmoid(x))
-    // Split tiles of the gather kernels finished inside the kernel
-    // (FinishSplitTile) instead of through `partial`: counters per
-    // [group][tile], slots [group * tiles + tile][split][BM * BN].
-    uint32_t* split_counters;
-    float* split_slots;
-};
-
-// The fused activation, each step rounded as the separate rows round it:
-// Relu is std::max(0.0f, v) (NaN maps to 0 like the reference Relu); SiLU is
-// the Sigmoid row's SigmoidF32(v) followed by the Mul row's product.
-__device__ __forceinline__ float Activate(int act, float v) {
-    if (act == 1) {
-        return (0.0f < v) ? v : 0.0f;
-    }
-    if (act == 2) {
-        return __fmul_rn(v, SigmoidF32(v));
-    }
-    return v;
-}
-
-__device__ __forceinline__ float Finish(const ConvArgs& p, float v, int64_t y_index) {
-    if (p.residual != nullptr) {
-        v = v + p.residual[y_index];
-    }
-    return Activate(p.act, v);
-}
 
 // Gathers B(k, n) = X_col for one K tile. Thread t owns column nn = t % BN for
 // every pass (the column decode happens once per block); rows are assigned
@@ -196,16 +139,6 @@ struct ConvBLoader {
 // clamped addresses, and no separate edge path. Requires both tensors under
 // 2 GiB (32-bit buffer offsets); the host checks.
 
-// Workgroups are dispatched round-robin over the 8 XCDs (workgroup i on XCD
-// i % 8), each with its own L2. Workgroup i of the first `count` rounded down
-// to a multiple of 8 takes tile (i % 8) * (whole / 8) + i / 8, so each XCD
-// works through one contiguous run of tiles, whose neighbours share operand
-// rows or columns in that XCD's L2; the rest keep their index.
-__device__ __forceinline__ int64_t XcdTile(int64_t i, int64_t count) {
-    const int64_t whole = count / 8 * 8;
-    return i < whole ? (i % 8) * (whole / 8) + i / 8 : i;
-}
-
 // For `count` = tiles_m * tiles_n tiles numbered row tile fastest, with
 // tiles_m a multiple of 8: workgroup i (on XCD i % 8) takes row tile
 // (i % 8) * (tiles_m / 8) + j % (tiles_m / 8) of column tile j / (tiles_m / 8),
@@ -216,19 +149,6 @@ __device__ __forceinline__ int64_t XcdTileByRow(int64_t i, int64_t count, int64_
     const int64_t j = i / 8;
     (void)count;
     return (i % 8) * per + j % per + tiles_m * (j / per);
-}
-
-constexpr uint32_t kBufferWord3 = 0x00020000; // raw 32-bit dword buffer (gfx9 family)
-constexpr uint32_t kOutOfRange = 0x80000000u; // >= every num_records used here
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t MakeRsrc(const float* base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), static_cast<short>(0),
-                                             static_cast<int>(bytes), static_cast<int>(kBufferWord3));
-}
-
-__device__ __forceinline__ float BufferLoad(__amdgpu_buffer_rsrc_t r, uint32_t voffset, uint32_t soffset) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, static_cast<int>(voffset),
-                                                                          static_cast<int>(soffset), 0));
 }
 
 // A tile (BM x BK, k-major in LDS) of the tap-major weight view:
@@ -1473,30 +1393,6 @@ bool HaloApplies(const ConvArgs& p) {
            p.s_h <= 2 * p.d_h + 1 && p.n_total < (int64_t{1} << 31) &&
            p.batch * p.c * p.plane_in * 4 < (int64_t{1} << 31) && p.m * p.kg * 4 < (int64_t{1} << 31) &&
            p.out_w < (1 << 16) && p.out_h < (1 << 16);
-}
-
-// ---- Per-geometry choice of a kernel configuration ----------------------------
-// (tune.hpp). Measured on ResNet-18 bs32: the best candidate is 3-6% ahead of
-// any fixed rule on the 3x3 layers, and the 1x1 stride-2 layers want small
-// tiles. The cache key is the geometry alone, so a Conv row and a FusedConv
-// row of the same geometry compute their sums the same way.
-using ConvKey = std::array<int64_t, 22>;
-
-ConvKey KeyOf(const ConvArgs& p) {
-    return ConvKey{p.batch, p.c,     p.m,     p.group, p.in_d, p.in_h, p.in_w, p.k_d, p.k_h, p.k_w, p.out_d,
-                   p.out_h, p.out_w, p.s_d,   p.s_h,   p.s_w,  p.d_d,  p.d_h,  p.d_w, p.p_d, p.p_h, p.p_w};
-}
-
-template <class Launch>
-int ChooseConvConfig(const char* family, std::map<ConvKey, int>& cache, const ConvArgs& p, hipStream_t stream,
-                     int count, int fallback, Launch launch) {
-    static std::mutex mu;
-    const size_t y_bytes = static_cast<size_t>(p.batch * p.m * p.plane_out) * sizeof(float);
-    return ChooseConfig(family, cache, mu, KeyOf(p), y_bytes, stream, count, fallback, [&](int i, float* scratch) {
-        ConvArgs q = p;
-        q.y = scratch;
-        return launch(i, q, stream);
-    });
 }
 
 // 3x3 candidates: tile shape i / 4 (0 W, 1 M, 2 Q, 3 N) with split-K count
@@ -2888,15 +2784,48 @@ ConvArgs MakeConvArgs(const float* x, const float* w, const float* bias, const f
     return p;
 }
 
+// Split-operand kernel (0) or fp32 kernels (1). With stride 1 and at least 32
+// channels per group the split one is ahead throughout (ResNet-18 bs32 layers
+// 51-57 us against 70-74 on an MI355X). With a stride a patch is two to four
+// times the pixels for the same products, and below 32 channels half of each
+// K step is zeros: there the lead changes with the geometry (64 -> 128
+// channels at 57 x 57, batch 5: 20.3 against 18 us; 64 -> 128 at 56 x 56,
+// batch 32: 37 against 44), and the two are timed.
+template <class Launch>
+int ChoosePath(const char* family, std::map<ConvKey, int>& chosen, const ConvArgs& p, hipStream_t s, Launch launch) {
+    if (p.k_h > 3 || p.k_w > 3 || p.cg < 16 || p.cg % 8 != 0) {
+        return 1;
+    }
+    if (const char* forced = std::getenv("NERT_HIP_CONV_CANDIDATE")) {
+        return std::atoi(forced) < 400 ? 1 : 0;
+    }
+    if (p.s_h == 1 && p.s_w == 1 && p.cg >= 32) {
+        return 0;
+    }
+    return ChooseConvConfig(family, chosen, p, s, 2, 0, launch);
+}
+
 // Runs one convolution on the fastest kernel that applies.
 void RunConv(const ConvArgs& p, hipStream_t s) {
     if (p.n_total == 0 || p.mg == 0) {
         return;
     }
-    if (TryPointwise(p, s) || TryPatchGemm(p, s) || TrySmallChannelConv(p, s) || TryHaloConv(p, s)) {
+    if (TryPointwise(p, s) || TryPatchGemm(p, s) || TrySmallChannelConv(p, s)) {
         return;
     }
-    LaunchGatherConv(p, s);
+    const auto fp32 = [](const ConvArgs& q, hipStream_t st) {
+        if (!TryHaloConv(q, st)) {
+            LaunchGatherConv(q, st);
+        }
+        return true;
+    };
+    static std::map<ConvKey, int> chosen;
+    const auto launch = [&fp32](int i, const ConvArgs& q, hipStream_t st) {
+        return i == 0 ? TrySplitConv(q, nullptr, st) : fp32(q, st);
+    };
+    if (!launch(ChoosePath("convpath", chosen, p, s, launch), p, s)) {
+        fp32(p, s);
+    }
 }
 
 } // namespace nert_hip
@@ -2937,11 +2866,21 @@ void RunConvPair(const ConvArgs& p, const float* w2, const float* bias2, float* 
         return;
     }
     hipStream_t s = StreamOr(stream);
-    if (TryHaloPair(p, HaloPair{w2, bias2, y2}, s)) {
-        return;
+    const ConvPair pair{w2, bias2, y2};
+    const auto fp32 = [&](const ConvArgs& q, hipStream_t st) {
+        if (!TryHaloPair(q, HaloPair{w2, bias2, y2}, st)) {
+            RunConv(q, st);
+            RunConv(p2, st);
+        }
+        return true;
+    };
+    static std::map<ConvKey, int> chosen;
+    const auto launch = [&](int i, const ConvArgs& q, hipStream_t st) {
+        return i == 0 ? TrySplitConv(q, &pair, st) : fp32(q, st);
+    };
+    if (!launch(ChoosePath("convpathpair", chosen, p, s, launch), p, s)) {
+        fp32(p, s);
     }
-    RunConv(p, s);
-    RunConv(p2, s);
 }
 
 } // namespace nert_hip
@@ -2953,6 +2892,21 @@ extern "C" int nert_hip_conv_pair_f32(const float* x, const float* w, const floa
         nert_hip::RunConvPair(nert_hip::MakeConvArgs(x, w, bias, residual, y, d, act), w2, bias2, y2, d, stream);
     });
 }
+
+namespace nert_hip {
+
+// A fused convolution, or (w2 set) a pair, with copies of its weights in
+// other orders.
+void RunPrepared(const ConvArgs& p, const float* w2, const float* bias2, float* y2, const nert_conv_desc* d,
+                 void* stream) {
+    if (w2 != nullptr) {
+        RunConvPair(p, w2, bias2, y2, d, stream);
+    } else {
+        RunConv(p, StreamOr(stream));
+    }
+}
+
+} // namespace nert_hip
 
 extern "C" int nert_hip_conv_packed_f32(const float* x, const float* w, const float* w_packed, const float* bias,
                                         const float* residual, float* y, const float* w2, const float* bias2,
@@ -2966,11 +2920,20 @@ extern "C" int nert_hip_conv_packed_f32(const float* x, const float* w, const fl
             throw nert_hip::Error("conv packed: packed weights need C / group to be a multiple of 8");
         }
         p.w_packed = w_packed;
-        if (w2 != nullptr) {
-            nert_hip::RunConvPair(p, w2, bias2, y2, d, stream);
-            return;
+        nert_hip::RunPrepared(p, w2, bias2, y2, d, stream);
+    });
+}
+
+extern "C" int nert_hip_conv_presplit_f32(const float* x, const float* w, const float* w_split, const float* bias,
+                                          const float* residual, float* y, const float* w2, const float* bias2,
+                                          float* y2, const nert_conv_desc* d, int act, void* stream) {
+    return nert_hip::Guard([&] {
+        nert_hip::ConvArgs p = nert_hip::MakeConvArgs(x, w, bias, residual, y, d, act);
+        if (w_split == nullptr || (reinterpret_cast<uintptr_t>(w_split) & 15) != 0) {
+            throw nert_hip::Error("conv presplit: the split weights are null or not 16-byte aligned");
         }
-        nert_hip::RunConv(p, nert_hip::StreamOr(stream));
+        p.w_split = w_split;
+        nert_hip::RunPrepared(p, w2, bias2, y2, d, stream);
     });
 }
 

@@ -1,0 +1,136 @@
+#pragma once
+// What the convolution kernels share: their arguments, the fused epilogue,
+// buffer addressing and the per-geometry choice.
+
+#include <array>
+#include <map>
+#include <mutex>
+
+#include "common.hpp"
+#include "tune.hpp"
+
+namespace nert_hip {
+
+struct ConvArgs {
+    const float* x;
+    const float* w;
+    // W again in the order the 3x3 LDS-patch kernel stores it, or null: per
+    // output channel, blocks of 8 input channels, in a block the taps, in a
+    // tap the 8 channels ([M][C_g / 8][KH * KW][8]); that kernel then copies
+    // it to LDS with 16-byte stores instead of transposing 4-byte ones.
+    // Every other kernel reads `w`.
+    const float* w_packed;
+    // W split for the kernel of conv_split.hip (nert_hip_conv_split_weights),
+    // or null; a pair's 1x1 weights, split, follow it.
+    const float* w_split;
+    const float* bias;
+    float* y;
+    int64_t batch, c, m, group;
+    int64_t cg, mg, kg; // channels per group, outputs per group, K per group
+    int32_t in_d, in_h, in_w;
+    int32_t k_d, k_h, k_w;
+    int32_t out_d, out_h, out_w;
+    int32_t s_d, s_h, s_w;
+    int32_t d_d, d_h, d_w;
+    int32_t p_d, p_h, p_w;
+    int64_t plane_out; // OD*OH*OW
+    int64_t plane_in;  // ID*IH*IW
+    int64_t n_total;   // batch * plane_out
+    FastDiv div_kvol, div_khw, div_kw;
+    int64_t k_per_split;
+    float* partial; // [splits][group][M_g][N] when split
+    // Optional epilogue (fused rows): y = act(acc + bias + residual), in that
+    // order, so the result equals Conv, then Add, then the activation rows
+    // bit for bit.
+    const float* residual; // same layout as y, or null
+    int32_t act;           // 0 none, 1 Relu, 2 SiLU (x * Sigmoid(x))
+    // Split tiles of the gather kernels finished inside the kernel
+    // (FinishSplitTile) instead of through `partial`: counters per
+    // [group][tile], slots [group * tiles + tile][split][BM * BN].
+    uint32_t* split_counters;
+    float* split_slots;
+};
+
+// The fused activation, each step rounded as the separate rows round it:
+// Relu is std::max(0.0f, v) (NaN maps to 0 like the reference Relu); SiLU is
+// the Sigmoid row's SigmoidF32(v) followed by the Mul row's product.
+__device__ __forceinline__ float Activate(int act, float v) {
+    if (act == 1) {
+        return (0.0f < v) ? v : 0.0f;
+    }
+    if (act == 2) {
+        return __fmul_rn(v, SigmoidF32(v));
+    }
+    return v;
+}
+
+__device__ __forceinline__ float Finish(const ConvArgs& p, float v, int64_t y_index) {
+    if (p.residual != nullptr) {
+        v = v + p.residual[y_index];
+    }
+    return Activate(p.act, v);
+}
+
+// Workgroups are dispatched round-robin over the 8 XCDs (workgroup i on XCD
+// i % 8), each with its own L2. Workgroup i of the first `count` rounded down
+// to a multiple of 8 takes tile (i % 8) * (whole / 8) + i / 8, so each XCD
+// works through one contiguous run of tiles, whose neighbours share operand
+// rows or columns in that XCD's L2; the rest keep their index.
+__device__ __forceinline__ int64_t XcdTile(int64_t i, int64_t count) {
+    const int64_t whole = count / 8 * 8;
+    return i < whole ? (i % 8) * (whole / 8) + i / 8 : i;
+}
+
+constexpr uint32_t kBufferWord3 = 0x00020000; // raw 32-bit dword buffer (gfx9 family)
+constexpr uint32_t kOutOfRange = 0x80000000u; // >= every num_records used here
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t MakeRsrc(const float* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), static_cast<short>(0),
+                                             static_cast<int>(bytes), static_cast<int>(kBufferWord3));
+}
+
+__device__ __forceinline__ float BufferLoad(__amdgpu_buffer_rsrc_t r, uint32_t voffset, uint32_t soffset) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, static_cast<int>(voffset),
+                                                                          static_cast<int>(soffset), 0));
+}
+
+// ---- Per-geometry choice of a kernel configuration ----------------------------
+// (tune.hpp). Measured on ResNet-18 bs32: the best candidate is 3-6% ahead of
+// any fixed rule on the 3x3 layers, and the 1x1 stride-2 layers want small
+// tiles. The cache key is the geometry alone, so a Conv row and a FusedConv
+// row of the same geometry compute their sums the same way.
+using ConvKey = std::array<int64_t, 22>;
+
+inline ConvKey KeyOf(const ConvArgs& p) {
+    return ConvKey{p.batch, p.c,     p.m,     p.group, p.in_d, p.in_h, p.in_w, p.k_d, p.k_h, p.k_w, p.out_d,
+                   p.out_h, p.out_w, p.s_d,   p.s_h,   p.s_w,  p.d_d,  p.d_h,  p.d_w, p.p_d, p.p_h, p.p_w};
+}
+
+template <class Launch>
+int ChooseConvConfig(const char* family, std::map<ConvKey, int>& cache, const ConvArgs& p, hipStream_t stream,
+                     int count, int fallback, Launch launch) {
+    static std::mutex mu;
+    const size_t y_bytes = static_cast<size_t>(p.batch * p.m * p.plane_out) * sizeof(float);
+    return ChooseConfig(family, cache, mu, KeyOf(p), y_bytes, stream, count, fallback, [&](int i, float* scratch) {
+        ConvArgs q = p;
+        q.y = scratch;
+        return launch(i, q, stream);
+    });
+}
+
+// A 1x1 convolution run with a 3x3 one of the same input, stride and output
+// shape (conv pairs): its weights, bias or null, and output; no activation.
+struct ConvPair {
+    const float* w2;
+    const float* bias2;
+    float* y2;
+};
+
+// Words (4 bytes) of split weights.
+int64_t SplitWeightWords(int64_t m, int64_t cg, int64_t taps, int64_t group);
+
+// Runs the convolution (and its pair, when given) on the split-operand
+// kernel of conv_split.hip; false when that kernel does not take it.
+bool TrySplitConv(const ConvArgs& p, const ConvPair* pair, hipStream_t stream);
+
+} // namespace nert_hip

@@ -1,0 +1,795 @@
+// Convolution on the bf16 matrix cores with all 24 bits of both operands
+// (split_mma.hpp), as an implicit GEMM whose K runs channel block by channel
+// block (32 channels) and, inside a block, tap by tap.
+//
+// What bounds it: the fp32 instruction's rate (153 TFLOP/s sustained) bounded
+// the LDS-patch kernel of conv.hip; six bf16 products take 2.7 times less
+// matrix time, and then LDS reads and the operand splits matter. So:
+//   - a workgroup copies the input patch of its pixels once per channel block
+//     and splits it once: the k_h * k_w taps read the same split pieces at
+//     shifted positions (a 3x3 splits each input element 1/9 as often as a
+//     GEMM of the same size would);
+//   - LDS holds a patch as [piece][channel octet][position], 16 bytes each, so
+//     the operand of 16 pixels x 32 channels is one ds_read_b128 and, within
+//     an image row, free of bank conflicts; at stride s the positions of a
+//     row are stored by residue mod s, so that also there consecutive pixels
+//     are consecutive slots;
+//   - the weights come split (nert_hip_conv_split_weights; a call without such
+//     a copy makes one in the workspace first) in the order of the operands,
+//     so a wave loads its rows of the next tap straight into registers: no
+//     LDS, and no barrier but where the patch changes, once in k_h * k_w steps.
+//
+// Pixels: the output plane is cut into strips of `sw` columns (one strip when
+// the whole width's patch fits LDS); a tile is BN consecutive pixels of one
+// strip, over its rows and images, so 7x7 and 14x14 planes waste no columns
+// of a tile.
+
+#include "conv_args.hpp"
+#include "split_mma.hpp"
+#include "../../include/nert_hip.h"
+
+#include <algorithm>
+#include <cmath>
+#include <cstdlib>
+#include <map>
+
+namespace nert_hip {
+namespace {
+
+constexpr int kSplitMaxKw = 8;
+
+struct SplitGeom {
+    int32_t taps;    // k_h * k_w
+    int32_t blocks;  // channel blocks of 32, the last zero-filled
+    int32_t sw;      // strip width
+    int32_t strips;
+    int32_t tiles_m; // row tiles of one group
+    int32_t total;   // pixels of one strip: batch * out_h * sw
+    int32_t seg;     // LDS slots per residue class of a patch row
+    int32_t row_slots; // LDS slots per patch row: ps_w * seg
+    int32_t positions; // LDS slots per octet plane
+    int32_t ps_h, ps_w;     // pixel steps in the patch
+    int32_t step_h, step_w; // input step of a patch position (1x1 convolutions copy only what they read)
+    int32_t halo;           // patch rows of one output row
+    int32_t rows_full;      // patch rows of a whole image
+    int32_t q_off[kSplitMaxKw]; // slot displacement of tap column q
+    int32_t tap_row;            // slot displacement of tap row 1
+    FastDiv div_plane; // by out_h * sw
+    FastDiv div_sw;
+    FastDiv div_row; // by row_slots
+    FastDiv div_seg;
+    FastDiv div_rows_full;
+    FastDiv div_pos; // by positions
+    // Workgroups [0, n_full) take tiles whole; the other tiles are cut into
+    // `pieces` runs of `piece_steps` K steps each, one workgroup per run, summed
+    // by the last one to finish (FinishSplitParts).
+    int32_t n_full;
+    int32_t rest;
+    int32_t pieces;
+    int32_t piece_steps;
+    uint32_t* counters; // per [group][rest tile]
+    float* slots;
+    int32_t vec; // four consecutive pixels are 16 aligned bytes of y (and residual)
+    // Paired 1x1 convolution: its tiles follow, one K step per channel block.
+    const float* w2;
+    const float* bias2;
+    float* y2;
+};
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_PER_SIMD>
+struct SplitTile {
+    static constexpr int kBM = BM;
+    static constexpr int kBN = BN;
+    static constexpr int kWavesM = WAVES_M;
+    static constexpr int kThreads = 64 * WAVES_M * WAVES_N;
+    static constexpr int kRows = BM / WAVES_M;
+    static constexpr int kCols = BN / WAVES_N;
+    static constexpr int kRB = kRows / 16;
+    static constexpr int kCB = kCols / 16;
+    static constexpr int kPerSimd = WAVES_PER_SIMD;
+    static_assert(kRows % 16 == 0 && kCols % 32 == 0, "wave tiles are whole pairs of 16 x 16 blocks");
+};
+
+// Split weights in memory, per group, 16-row block, channel block and tap:
+// [piece][64 slots], slot l of 16 bytes being row l % 16, channel octet l / 16.
+constexpr int kSplitBlockWords = 3 * 64 * 4;
+
+// NPOS: patch octets (8 channels of one position) per thread.
+template <class Tile, int NPOS>
+__global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void SplitConvKernel(ConvArgs p, SplitGeom h) {
+    constexpr int T = Tile::kThreads;
+    constexpr int BM = Tile::kBM;
+    constexpr int RB = Tile::kRB;
+    constexpr int CB = Tile::kCB;
+    extern __shared__ __attribute__((aligned(16))) uint32_t xbuf[];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_row = (wave % Tile::kWavesM) * Tile::kRows;
+    const int wave_col = (wave / Tile::kWavesM) * Tile::kCols;
+    const int g = blockIdx.y;
+
+    // This workgroup's tile and its run of K steps.
+    const int id = blockIdx.x;
+    const int split_end = h.n_full + h.rest * h.pieces;
+    int tile;
+    int part = -1;
+    bool paired = false;
+    int ntaps = h.taps;
+    int s_begin = 0;
+    int s_end = h.blocks * h.taps;
+    if (id < h.n_full) {
+        tile = static_cast<int>(XcdTile(id, h.n_full));
+    } else if (id < split_end) {
+        const int q = id - h.n_full;
+        tile = h.n_full + q / h.pieces;
+        part = q % h.pieces;
+        s_begin = part * h.piece_steps;
+        s_end = min(s_begin + h.piece_steps, s_end);
+    } else {
+        tile = id - split_end;
+        paired = true;
+        ntaps = 1;
+        s_end = h.blocks;
+    }
+    const int row0 = (tile % h.tiles_m) * BM;
+    const int pt = tile / h.tiles_m;
+    const int strip = pt % h.strips;
+    const int col0 = pt / h.strips * Tile::kBN;
+
+    // The tile's first and last pixels: image and output row of each.
+    uint32_t rem;
+    const int b_first = static_cast<int>(DivMod(h.div_plane, static_cast<uint32_t>(col0), rem));
+    const int oh_first = static_cast<int>(h.div_sw.Div(rem));
+    const int b_last =
+        static_cast<int>(DivMod(h.div_plane, static_cast<uint32_t>(min(col0 + Tile::kBN, h.total) - 1), rem));
+    const int oh_last = static_cast<int>(h.div_sw.Div(rem));
+    const int run0_end = b_last == b_first ? oh_last : p.out_h - 1;
+    const int rows0 = (run0_end - oh_first) * h.ps_h + h.halo; // patch rows of the first image
+
+    // Patch octets this thread copies: item e = tid + i * T is octet
+    // e / positions of position e % positions, at LDS slot e.
+    const __amdgpu_buffer_rsrc_t xr = MakeRsrc(p.x, static_cast<uint32_t>(p.batch * p.c * p.plane_in * 4));
+    const uint32_t plane_bytes = static_cast<uint32_t>(p.plane_in * 4);
+    const int items = 4 * h.positions;
+    uint32_t xoff[NPOS];
+    int xoct[NPOS];
+#pragma unroll
+    for (int i = 0; i < NPOS; ++i) {
+        const int e = tid + i * T;
+        uint32_t off = kOutOfRange;
+        uint32_t pos;
+        xoct[i] = static_cast<int>(DivMod(h.div_pos, static_cast<uint32_t>(e), pos));
+        if (e < items) {
+            uint32_t in_row;
+            const int r = static_cast<int>(DivMod(h.div_row, pos, in_row));
+            uint32_t at;
+            const int residue = static_cast<int>(DivMod(h.div_seg, in_row, at));
+            const int x = static_cast<int>(at) * h.ps_w + residue;
+            int image = 0;
+            int local = r;
+            if (r >= rows0) {
+                uint32_t lr;
+                image = 1 + static_cast<int>(DivMod(h.div_rows_full, static_cast<uint32_t>(r - rows0), lr));
+                local = static_cast<int>(lr);
+            }
+            const int b = b_first + image;
+            const int ih = ((image == 0 ? oh_first : 0) * h.ps_h + local) * h.step_h - p.p_h;
+            const int iw = (strip * h.sw * h.ps_w + x) * h.step_w - p.p_w;
+            if (b <= b_last && ih >= 0 && ih < p.in_h && iw >= 0 && iw < p.in_w) {
+                off = static_cast<uint32_t>(((static_cast<int64_t>(b) * p.c + static_cast<int64_t>(g) * p.cg +
+                                              8 * xoct[i]) *
+                                                 p.plane_in +
+                                             ih * p.in_w + iw) *
+                                            4);
+            }
+        }
+        xoff[i] = off;
+    }
+
+    // Weights: the wave's row blocks are block_words apart.
+    const int block_bytes = h.blocks * ntaps * kSplitBlockWords * 4;
+    const int row_blocks = static_cast<int>((p.mg + 15) / 16);
+    const __amdgpu_buffer_rsrc_t wr =
+        MakeRsrc(p.w_split + (paired ? static_cast<int64_t>(row_blocks) * h.blocks * h.taps * kSplitBlockWords : 0),
+                 static_cast<uint32_t>(p.group) * row_blocks * block_bytes);
+    // (Rows past the last block read what follows or zero; they are not stored.)
+    const uint32_t w_wave = static_cast<uint32_t>(g * row_blocks + (row0 + wave_row) / 16) * block_bytes;
+
+    float xv[NPOS][8];
+    auto load_x = [&](int cb) {
+        const uint32_t base = static_cast<uint32_t>(cb) * 32u * plane_bytes;
+        const int octets = static_cast<int>(p.cg / 8) - 4 * cb; // of this block
+#pragma unroll
+        for (int i = 0; i < NPOS; ++i) {
+            const uint32_t off = xoct[i] < octets ? xoff[i] : kOutOfRange;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                xv[i][c] = BufferLoad(xr, off, base + static_cast<uint32_t>(c) * plane_bytes);
+            }
+        }
+    };
+    auto store_x = [&]() {
+#pragma unroll
+        for (int i = 0; i < NPOS; ++i) {
+            const int e = tid + i * T;
+            if (e < items) {
+                const SplitOctet o = Split8(nert_floatx4{xv[i][0], xv[i][1], xv[i][2], xv[i][3]},
+                                            nert_floatx4{xv[i][4], xv[i][5], xv[i][6], xv[i][7]});
+#pragma unroll
+                for (int piece = 0; piece < 3; ++piece) {
+                    *reinterpret_cast<nert_uintx4*>(xbuf + (piece * items + e) * 4) = o.piece[piece];
+                }
+            }
+        }
+    };
+    // Operand slots of this lane: the patch position of the window origin of
+    // its pixel of every column block.
+    int frag_x[CB];
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+        const int n = col0 + wave_col + 16 * j + (lane & 15);
+        int pos = 0; // pixels past the end read position 0; their sums are never stored
+        if (n < h.total) {
+            const int b = static_cast<int>(DivMod(h.div_plane, static_cast<uint32_t>(n), rem));
+            uint32_t x;
+            const int oh = static_cast<int>(DivMod(h.div_sw, rem, x));
+            const int image = b - b_first;
+            const int start = image == 0 ? 0 : rows0 + (image - 1) * h.rows_full;
+            pos = (start + (oh - (image == 0 ? oh_first : 0)) * h.ps_h) * h.row_slots + static_cast<int>(x);
+        }
+        frag_x[j] = ((lane >> 4) * h.positions + pos) * 4;
+    }
+
+    SplitAccum<RB, CB> acc;
+    acc.Zero();
+    // A step's place: channel block, tap and the tap's row and column.
+    struct Place {
+        int cb, t, r, q;
+    };
+    auto place = [&](int s) {
+        Place w;
+        w.cb = s / ntaps;
+        w.t = s % ntaps;
+        w.r = w.t / p.k_w;
+        w.q = w.t % p.k_w;
+        return w;
+    };
+    auto advance = [&](Place& w) {
+        ++w.t;
+        ++w.q;
+        if (w.q == p.k_w) {
+            w.q = 0;
+            ++w.r;
+        }
+        if (w.t == ntaps) {
+            w = Place{w.cb + 1, 0, 0, 0};
+        }
+    };
+    nert_uintx4 row[RB][3];
+    nert_uintx4 col[CB][3];
+    auto load_row = [&](int i, const Place& w) {
+        const uint32_t base = w_wave + static_cast<uint32_t>(i * block_bytes + (w.cb * ntaps + w.t) * kSplitBlockWords * 4);
+#pragma unroll
+        for (int piece = 0; piece < 3; ++piece) {
+            row[i][piece] =
+                __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16 + piece * 1024, static_cast<int>(base), 0);
+        }
+    };
+    // The tap a paired 1x1 reads is the 3x3's centre.
+    const int pair_off = h.tap_row + h.q_off[1];
+    auto displacement = [&](const Place& w) { return paired ? pair_off : w.r * h.tap_row + h.q_off[w.q]; };
+    auto load_col = [&](int j, int toff) {
+#pragma unroll
+        for (int piece = 0; piece < 3; ++piece) {
+            col[j][piece] = *reinterpret_cast<const nert_uintx4*>(xbuf + piece * items * 4 + frag_x[j] + toff * 4);
+        }
+    };
+    // One tap: two column blocks by one row block at a time, every operand
+    // replaced by the next tap's right after its last use. (Across a patch
+    // change the columns read here are stale and are read again.)
+    auto step = [&](const Place& next) {
+        const int toff = displacement(next);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+#pragma unroll
+            for (int j = 0; j < CB; j += 2) {
+                acc.StepPair(i, j, row[i], col);
+                if (i == RB - 1) {
+                    load_col(j, toff);
+                    load_col(j + 1, toff);
+                }
+                if (j == CB - 2) {
+                    load_row(i, next);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    if (s_begin < s_end) {
+        Place now = place(s_begin);
+        const int last_cb = (s_end - 1) / ntaps;
+        load_x(now.cb);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            load_row(i, now);
+        }
+        int s = s_begin;
+        auto run_step = [&]() {
+            Place next = now;
+            if (++s < s_end) {
+                advance(next);
+            }
+            step(next);
+            now = next;
+        };
+        while (true) {
+            store_x();
+            __syncthreads();
+            if (now.cb < last_cb) {
+                load_x(now.cb + 1);
+            }
+            const int toff = displacement(now);
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+                load_col(j, toff);
+            }
+            // The block's first step stands outside the loop: its weights were
+            // requested before the patch loads above, so it need not wait for
+            // those; every later step's weights come behind them.
+            const int in_block = min(ntaps - now.t, s_end - s);
+            run_step();
+            for (int k = 1; k < in_block; ++k) {
+                run_step();
+            }
+            __syncthreads(); // every wave is done with the patch
+            if (s >= s_end) {
+                break;
+            }
+        }
+    }
+    if (acc.Finish()) {
+        // Non-finite or huge values: the block again in float32, k = step * 32
+        // + channel of the block.
+        auto row = [&](int i, int64_t k) -> float {
+            const int64_t m = row0 + wave_row + 16 * i + (lane & 15);
+            const Place w = place(static_cast<int>(k / 32));
+            const int64_t c = w.cb * 32 + k % 32;
+            if (m >= p.mg || c >= p.cg) {
+                return 0.0f;
+            }
+            return paired ? h.w2[m * p.cg + c] : p.w[((g * p.mg + m) * p.cg + c) * ntaps + w.t];
+        };
+        auto col = [&](int j, int64_t k) -> float {
+            const int n = col0 + wave_col + 16 * j + (lane & 15);
+            const Place w = place(static_cast<int>(k / 32));
+            const int64_t c = w.cb * 32 + k % 32;
+            if (n >= h.total || c >= p.cg) {
+                return 0.0f;
+            }
+            uint32_t left;
+            const int b = static_cast<int>(DivMod(h.div_plane, static_cast<uint32_t>(n), left));
+            uint32_t x;
+            const int oh = static_cast<int>(DivMod(h.div_sw, left, x));
+            const int ih = oh * p.s_h - p.p_h + (paired ? 1 : w.r) * p.d_h;
+            const int iw = (strip * h.sw + static_cast<int>(x)) * p.s_w - p.p_w + (paired ? 1 : w.q) * p.d_w;
+            if (ih < 0 || ih >= p.in_h || iw < 0 || iw >= p.in_w) {
+                return 0.0f;
+            }
+            return p.x[((static_cast<int64_t>(b) * p.c + static_cast<int64_t>(g) * p.cg + c) * p.in_h + ih) * p.in_w + iw];
+        };
+        RerunFloat32(acc, static_cast<int64_t>(s_begin) * 32, static_cast<int64_t>(s_end) * 32, row, col);
+    }
+    if (part >= 0) {
+        const int64_t t = static_cast<int64_t>(g) * h.rest + (tile - h.n_full);
+        if (!FinishSplitParts<RB, CB, T, double>(acc, h.slots + t * h.pieces * BM * Tile::kBN, h.counters + t, part,
+                                                 h.pieces, reinterpret_cast<int*>(xbuf))) {
+            return;
+        }
+    }
+
+    // y = act(sum + bias + residual), each step rounded as the separate rows
+    // round it. A lane holds four consecutive pixels of one output channel.
+    float* const y = paired ? h.y2 : p.y;
+    const float* const bias = paired ? h.bias2 : p.bias;
+    const float* const residual = paired ? nullptr : p.residual;
+    const int act = paired ? 0 : p.act;
+    float bv[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+        const int64_t m = row0 + wave_row + 16 * i + (lane & 15);
+        bv[i] = bias != nullptr && m < p.mg ? bias[g * p.mg + m] : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+        int64_t at[4];
+        bool ok[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int n = col0 + wave_col + 16 * j + 4 * (lane >> 4) + v;
+            const int b = static_cast<int>(DivMod(h.div_plane, static_cast<uint32_t>(n), rem));
+            uint32_t x;
+            const int oh = static_cast<int>(DivMod(h.div_sw, rem, x));
+            const int ow = strip * h.sw + static_cast<int>(x);
+            ok[v] = n < h.total && ow < p.out_w;
+            at[v] = ok[v] ? (static_cast<int64_t>(b) * p.m + g * p.mg) * p.plane_out +
+                                static_cast<int64_t>(oh) * p.out_w + ow
+                          : 0;
+        }
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const int64_t m = row0 + wave_row + 16 * i + (lane & 15);
+            if (m >= p.mg) {
+                continue;
+            }
+            nert_floatx4 value = acc.big[i][j];
+            if (h.vec != 0) {
+                if (!ok[0]) {
+                    continue;
+                }
+                const int64_t y_at = at[0] + m * p.plane_out;
+                if (bias != nullptr) {
+                    value = value + bv[i];
+                }
+                if (residual != nullptr) {
+                    value = value + *reinterpret_cast<const nert_floatx4*>(residual + y_at);
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    value[v] = Activate(act, value[v]);
+                }
+                *reinterpret_cast<nert_floatx4*>(y + y_at) = value;
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    if (ok[v]) {
+                        const int64_t y_at = at[v] + m * p.plane_out;
+                        float f = value[v];
+                        if (bias != nullptr) {
+                            f = f + bv[i];
+                        }
+                        if (residual != nullptr) {
+                            f = f + residual[y_at];
+                        }
+                        y[y_at] = Activate(act, f);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// ---- Launch -------------------------------------------------------------------
+
+constexpr int kLdsPerCu = 160 * 1024;
+constexpr int kCUs = 256;
+
+template <class Tile, int NPOS>
+void LaunchSplitKernel(const ConvArgs& p, const SplitGeom& h, dim3 grid, int lds, hipStream_t stream) {
+    constexpr auto kernel = SplitConvKernel<Tile, NPOS>;
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu);
+    Check(raised, "hipFuncSetAttribute(SplitConvKernel)");
+    kernel<<<grid, Tile::kThreads, lds, stream>>>(p, h);
+    CheckLaunch("SplitConvKernel launch");
+}
+
+// The patch of a tile of BN pixels in strips of width sw.
+struct PatchSize {
+    int64_t row_slots, positions;
+    int32_t seg;
+};
+
+template <int BN>
+PatchSize SizePatch(const ConvArgs& p, const SplitGeom& h, int64_t sw) {
+    const int64_t width = (sw - 1) * h.ps_w + (p.k_w - 1) * p.d_w + 1;
+    PatchSize s{};
+    s.seg = static_cast<int32_t>((width + h.ps_w - 1) / h.ps_w);
+    s.row_slots = static_cast<int64_t>(s.seg) * h.ps_w;
+    // Tiles start at multiples of BN: where the width divides BN or BN the
+    // width they start and end with a row.
+    const int64_t plane = sw * p.out_h;
+    int64_t rows = BN % sw == 0 ? BN / sw : sw % BN == 0 ? 1 : (BN - 1 + sw - 1) / sw + 1;
+    int64_t images = BN % plane == 0 ? BN / plane : plane % BN == 0 ? 1 : (BN - 1 + plane - 1) / plane + 1;
+    images = std::min<int64_t>(images, p.batch);
+    rows = std::min<int64_t>(rows, images * p.out_h);
+    // An image's run of r output rows takes r * ps_h + (halo - ps_h) patch rows.
+    const int64_t extra = h.halo - h.ps_h;
+    // Whole 16-slot groups (256 bytes, all banks): the lanes of two octets that
+    // LDS serves together then never share a bank.
+    s.positions = ((rows * h.ps_h + (extra > 0 ? images : 1) * extra) * s.row_slots + 15) / 16 * 16;
+    return s;
+}
+
+template <class Tile, int NPOS>
+bool TrySplitTile(const ConvArgs& p, const ConvPair* pair, int split, hipStream_t stream) {
+    SplitGeom h{};
+    const bool pointwise = p.k_h == 1 && p.k_w == 1;
+    h.taps = p.k_h * p.k_w;
+    h.blocks = static_cast<int32_t>((p.cg + 31) / 32);
+    h.step_h = pointwise ? p.s_h : 1;
+    h.step_w = pointwise ? p.s_w : 1;
+    h.ps_h = pointwise ? 1 : p.s_h;
+    h.ps_w = pointwise ? 1 : p.s_w;
+    h.halo = (p.k_h - 1) * p.d_h + 1;
+    h.rows_full = (p.out_h - 1) * h.ps_h + h.halo;
+    // Strip count: the one with the least padding of the last strip plus
+    // patch copied per pixel, among those whose patch fits a thread's NPOS
+    // octets and LDS; half of LDS is worth a fifth (two workgroups per CU).
+    double best = 1e30;
+    for (int strips = 1; strips <= std::min(p.out_w, 64); ++strips) {
+        int64_t sw = (p.out_w + strips - 1) / strips;
+        if (strips > 1 && p.out_w % 4 == 0) {
+            sw = (sw + 3) / 4 * 4;
+        }
+        if ((p.out_w + sw - 1) / sw != strips) {
+            continue;
+        }
+        const PatchSize s = SizePatch<Tile::kBN>(p, h, sw);
+        const int64_t lds = s.positions * 192;
+        if (4 * s.positions > NPOS * Tile::kThreads || lds > kLdsPerCu) {
+            continue;
+        }
+        const double cost = static_cast<double>(strips * sw) / p.out_w *
+                            (1.0 + 0.05 * static_cast<double>(s.positions) / Tile::kBN) *
+                            (Tile::kThreads <= 256 && lds > kLdsPerCu / 2 ? 1.2 : 1.0);
+        if (cost < best) {
+            best = cost;
+            h.strips = strips;
+            h.sw = static_cast<int32_t>(sw);
+            h.seg = s.seg;
+            h.row_slots = static_cast<int32_t>(s.row_slots);
+            h.positions = static_cast<int32_t>(s.positions);
+        }
+    }
+    if (h.strips == 0) {
+        return false;
+    }
+    const int64_t total = p.batch * p.out_h * static_cast<int64_t>(h.sw);
+    const int64_t tiles_n = (total + Tile::kBN - 1) / Tile::kBN;
+    h.tiles_m = static_cast<int32_t>((p.mg + Tile::kBM - 1) / Tile::kBM);
+    const int64_t tiles = h.tiles_m * tiles_n * h.strips;
+    if (total + Tile::kBN >= (int64_t{1} << 31) || tiles * 16 >= (int64_t{1} << 31)) {
+        return false;
+    }
+    h.total = static_cast<int32_t>(total);
+    for (int q = 0; q < p.k_w; ++q) {
+        h.q_off[q] = (q * p.d_w) % h.ps_w * h.seg + (q * p.d_w) / h.ps_w;
+    }
+    h.tap_row = p.d_h * h.row_slots;
+    h.div_plane = FastDiv::Make(static_cast<uint32_t>(p.out_h * h.sw));
+    h.div_sw = FastDiv::Make(static_cast<uint32_t>(h.sw));
+    h.div_row = FastDiv::Make(static_cast<uint32_t>(h.row_slots));
+    h.div_seg = FastDiv::Make(static_cast<uint32_t>(h.seg));
+    h.div_rows_full = FastDiv::Make(static_cast<uint32_t>(h.rows_full));
+    h.div_pos = FastDiv::Make(static_cast<uint32_t>(h.positions));
+    const int lds = h.positions * 192;
+
+    // Splitting: with fewer tiles than a round of workgroups every tile is cut
+    // so that they fill it once; with more, the tiles of the last, partly empty
+    // round are. A round is what the chip holds (split 1) or one per CU
+    // (split 2: an uneven number of tiles per CU costs as much as an empty one).
+    const int by_regs = Tile::kPerSimd * 256 / Tile::kThreads;
+    const int64_t resident =
+        static_cast<int64_t>(kCUs) * (split == 2 ? 1 : std::max(1, std::min(by_regs, kLdsPerCu / lds)));
+    const int steps = h.blocks * h.taps;
+    h.n_full = static_cast<int32_t>(tiles);
+    h.rest = 0;
+    h.pieces = 1;
+    h.piece_steps = steps;
+    if (split != 0) {
+        constexpr int kMinSteps = 5;
+        const int most = std::min(steps / kMinSteps, split == 2 ? 6 : 16);
+        const int64_t all = tiles * p.group;
+        int pieces = 1;
+        int64_t rest = 0;
+        if (all * 2 <= resident) {
+            pieces = static_cast<int>(std::min<int64_t>(resident / all, most));
+            rest = tiles;
+        } else if (all > resident && p.group == 1) {
+            rest = all % resident;
+            double round = 1.0;
+            for (int q = 2; q <= most; ++q) {
+                const double r = std::ceil(static_cast<double>(rest * q) / static_cast<double>(resident)) / q;
+                if (r < round - 1e-9) {
+                    round = r;
+                    pieces = q;
+                }
+            }
+        }
+        if (pieces < 2 || rest == 0) {
+            return false;
+        }
+        h.counters = TileCounters(rest * p.group);
+        if (h.counters == nullptr) {
+            return false;
+        }
+        h.piece_steps = (steps + pieces - 1) / pieces;
+        h.pieces = (steps + h.piece_steps - 1) / h.piece_steps;
+        h.rest = static_cast<int32_t>(rest);
+        h.n_full = static_cast<int32_t>(tiles - rest);
+        h.slots = static_cast<float*>(Workspace(
+            rest * p.group * h.pieces * Tile::kBM * Tile::kBN * static_cast<int64_t>(sizeof(float)), stream));
+    }
+    const bool pitch = (p.out_w % 4 == 0 && h.sw % 4 == 0) || (h.strips == 1 && p.plane_out % 4 == 0);
+    auto aligned = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    h.vec = pitch && aligned(p.y) && aligned(p.residual) && (pair == nullptr || aligned(pair->y2));
+    int64_t grid_x = h.n_full + static_cast<int64_t>(h.rest) * h.pieces;
+    if (pair != nullptr) {
+        h.w2 = pair->w2;
+        h.bias2 = pair->bias2;
+        h.y2 = pair->y2;
+        grid_x += tiles;
+    }
+    const dim3 grid(static_cast<unsigned>(grid_x), static_cast<unsigned>(p.group), 1);
+    LaunchSplitKernel<Tile, NPOS>(p, h, grid, lds, stream);
+    return true;
+}
+
+template <class Tile, int LOW, int HIGH>
+bool TrySplitShape(const ConvArgs& p, const ConvPair* pair, int split, hipStream_t stream) {
+    return TrySplitTile<Tile, LOW>(p, pair, split, stream) || TrySplitTile<Tile, HIGH>(p, pair, split, stream);
+}
+
+// Candidate i: tile shape i / 3; i % 3 how tiles are cut along K (TrySplitTile).
+constexpr int kSplitConvCandidates = 21;
+
+bool LaunchSplitCandidate(int i, const ConvArgs& p, const ConvPair* pair, hipStream_t stream) {
+    const int split = i % 3;
+    switch (i / 3) {
+    case 0:
+        return TrySplitShape<SplitTile<64, 128, 2, 2, 2>, 4, 6>(p, pair, split, stream);
+    case 1:
+        return TrySplitShape<SplitTile<128, 128, 4, 2, 2>, 2, 3>(p, pair, split, stream);
+    case 2:
+        return TrySplitShape<SplitTile<128, 64, 4, 1, 2>, 3, 6>(p, pair, split, stream);
+    case 3:
+        return TrySplitShape<SplitTile<64, 64, 2, 2, 3>, 3, 6>(p, pair, split, stream);
+    case 4:
+        return TrySplitShape<SplitTile<32, 128, 1, 4, 3>, 4, 6>(p, pair, split, stream);
+    case 5:
+        return TrySplitShape<SplitTile<64, 256, 2, 4, 2>, 3, 4>(p, pair, split, stream);
+    default:
+        return TrySplitShape<SplitTile<32, 64, 2, 2, 3>, 3, 6>(p, pair, split, stream);
+    }
+}
+
+// 2-D convolutions with at least 16 channels per group in whole octets, whose
+// input and weights 32-bit buffer offsets reach. (Below 16 channels half or
+// more of every 32-deep step would be zeros.)
+bool SplitApplies(const ConvArgs& p, const ConvPair* pair) {
+    const bool three = p.k_h == 3 && p.k_w == 3;
+    const bool point = p.k_h == 1 && p.k_w == 1 && p.d_h == 1 && p.d_w == 1;
+    return p.k_d == 1 && p.in_d == 1 && p.out_d == 1 && (three || point) && p.cg >= 16 && p.cg % 8 == 0 &&
+           p.s_h >= 1 && p.s_w >= 1 && p.d_h >= 1 && p.d_w >= 1 && p.mg < (1 << 24) &&
+           p.batch * p.c * p.plane_in * 4 < (int64_t{1} << 31) && p.m * p.kg * 4 < (int64_t{1} << 31) &&
+           p.out_w < (1 << 16) && p.out_h < (1 << 16) && p.in_w < (1 << 16) && p.in_h < (1 << 16) &&
+           SplitWeightWords(p.m, p.cg, p.k_h * p.k_w, p.group) * 4 < (int64_t{1} << 31) &&
+           (pair == nullptr ||
+            (three && p.group == 1 && p.d_h == 1 && p.d_w == 1 && p.p_h == 1 && p.p_w == 1));
+}
+
+// Splits W [M][C_g][taps] into the order above, one 16-byte slot of the three
+// pieces per thread; rows and channels past W are zero.
+__global__ __launch_bounds__(256) void SplitWeightsKernel(const float* __restrict__ w, uint32_t* __restrict__ out,
+                                                          int mg, int cg, int taps, int row_blocks, int blocks,
+                                                          int64_t slots) {
+    const int64_t id = blockIdx.x * int64_t{256} + threadIdx.x;
+    if (id >= slots) {
+        return;
+    }
+    const int lane = static_cast<int>(id & 63);
+    int64_t at = id >> 6; // ((group * row_blocks + row block) * blocks + block) * taps + tap
+    const int64_t base = at * kSplitBlockWords + lane * 4;
+    const int t = static_cast<int>(at % taps);
+    at /= taps;
+    const int cb = static_cast<int>(at % blocks);
+    at /= blocks;
+    const int row = static_cast<int>(at % row_blocks) * 16 + lane % 16;
+    const int64_t g = at / row_blocks;
+    const int c0 = cb * 32 + lane / 16 * 8;
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        f[e] = row < mg && c0 + e < cg ? w[((g * mg + row) * cg + c0 + e) * taps + t] : 0.0f;
+    }
+    const SplitOctet o = Split8(nert_floatx4{f[0], f[1], f[2], f[3]}, nert_floatx4{f[4], f[5], f[6], f[7]});
+#pragma unroll
+    for (int piece = 0; piece < 3; ++piece) {
+        *reinterpret_cast<nert_uintx4*>(out + base + piece * 256) = o.piece[piece];
+    }
+}
+
+void SplitWeightsTo(const float* w, float* out, int64_t m, int64_t cg, int64_t taps, int64_t group,
+                    hipStream_t stream) {
+    const int64_t slots = SplitWeightWords(m, cg, taps, group) / 12;
+    SplitWeightsKernel<<<static_cast<unsigned>((slots + 255) / 256), 256, 0, stream>>>(
+        w, reinterpret_cast<uint32_t*>(out), static_cast<int>(m / group), static_cast<int>(cg),
+        static_cast<int>(taps), static_cast<int>((m / group + 15) / 16), static_cast<int>((cg + 31) / 32), slots);
+    CheckLaunch("SplitWeightsKernel launch");
+}
+
+// Gives a call without split weights a copy in workspace slot 1. False when
+// that would have to grow while the stream is captured.
+bool SplitInWorkspace(ConvArgs& p, const ConvPair* pair, hipStream_t stream) {
+    if (p.w_split != nullptr) {
+        return true;
+    }
+    const int64_t taps = p.k_h * p.k_w;
+    const int64_t main_words = SplitWeightWords(p.m, p.cg, taps, p.group);
+    const int64_t bytes = 4 * (main_words + (pair != nullptr ? SplitWeightWords(p.m, p.cg, 1, p.group) : 0));
+    if (!WorkspaceHolds(bytes, 1)) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        Check(hipStreamIsCapturing(stream, &capture), "hipStreamIsCapturing");
+        if (capture != hipStreamCaptureStatusNone) {
+            return false;
+        }
+    }
+    auto* const out = static_cast<float*>(Workspace(bytes, stream, 1));
+    SplitWeightsTo(p.w, out, p.m, p.cg, taps, p.group, stream);
+    if (pair != nullptr) {
+        SplitWeightsTo(pair->w2, out + main_words, p.m, p.cg, 1, p.group, stream);
+    }
+    p.w_split = out;
+    return true;
+}
+
+} // namespace
+
+int64_t SplitWeightWords(int64_t m, int64_t cg, int64_t taps, int64_t group) {
+    return group * ((m / group + 15) / 16) * ((cg + 31) / 32) * taps * kSplitBlockWords;
+}
+
+bool TrySplitConv(const ConvArgs& call, const ConvPair* pair, hipStream_t stream) {
+    if (!SplitApplies(call, pair)) {
+        return false;
+    }
+    ConvArgs p = call;
+    // NERT_HIP_CONV_CANDIDATE=400 + i forces candidate i where it fits.
+    if (const char* forced = std::getenv("NERT_HIP_CONV_CANDIDATE")) {
+        const int i = std::atoi(forced) - 400;
+        if (!SplitInWorkspace(p, pair, stream)) {
+            return false;
+        }
+        if (i >= 0 && i < kSplitConvCandidates && LaunchSplitCandidate(i, p, pair, stream)) {
+            return true;
+        }
+    }
+    if (!SplitInWorkspace(p, pair, stream)) {
+        return false;
+    }
+    static std::map<ConvKey, int> chosen;
+    const int fallback = p.mg <= 32 ? 12 : 9;
+    // The choice is the single convolution's also for a pair, so both compute
+    // the same sums.
+    const int c = ChooseConvConfig("convsplit", chosen, p, stream, kSplitConvCandidates, fallback,
+                                   [](int i, const ConvArgs& q, hipStream_t st) {
+                                       return LaunchSplitCandidate(i, q, nullptr, st);
+                                   });
+    return LaunchSplitCandidate(c, p, pair, stream) || LaunchSplitCandidate(9, p, pair, stream);
+}
+
+} // namespace nert_hip
+
+extern "C" {
+
+int64_t nert_hip_conv_split_words(int64_t m, int64_t cg, int64_t taps, int64_t group) {
+    return nert_hip::SplitWeightWords(m, cg, taps, group);
+}
+
+int nert_hip_conv_split_weights(const float* w, float* out, int64_t m, int64_t cg, int64_t taps, int64_t group,
+                                void* stream) {
+    return nert_hip::Guard([&] {
+        if (group <= 0 || m <= 0 || cg <= 0 || taps <= 0 || m % group != 0 || m >= (1 << 24) || cg >= (1 << 24) ||
+            taps >= (1 << 16)) {
+            throw nert_hip::Error("conv split weights: invalid shape");
+        }
+        if (nert_hip::SplitWeightWords(m, cg, taps, group) / 3072 >= (int64_t{1} << 31) - 1) {
+            throw nert_hip::Error("conv split weights: too many weights");
+        }
+        nert_hip::SplitWeightsTo(w, out, m, cg, taps, group, nert_hip::StreamOr(stream));
+    });
+}
+
+} // extern "C"

@@ -546,15 +546,36 @@ const float* PackedWeights(const std::string& context, const TensorView& w, cons
     return static_cast<const float*>(packed.data);
 }
 
+// The split copy of W (FusedConv's eighth input) and, in a pair, of W2 behind
+// it: float32 words in nert_hip_conv_split_weights' order.
+const float* SplitWeights(const std::string& context, const TensorView& split, const nert_conv_desc& d, bool paired) {
+    const int64_t cg = d.in_channels / d.group;
+    int64_t words =
+        nert_hip_conv_split_words(d.out_channels, cg, d.kernel[0] * d.kernel[1] * d.kernel[2], d.group);
+    if (paired) {
+        words += nert_hip_conv_split_words(d.out_channels, cg, 1, d.group);
+    }
+    if (split.dtype != DataType::Float32 || split.dims != std::vector<int64_t>{words}) {
+        throw InferenceException(context + ": the split weights must be float32 [" + std::to_string(words) + "]");
+    }
+    if (split.data == nullptr) {
+        throw InferenceException(context + ": null buffer");
+    }
+    return static_cast<const float*>(split.data);
+}
+
+// Whether FusedConv input `i` is there.
+bool HasInput(const Views& inputs, size_t i) { return inputs.size() > i && inputs[i].dtype != DataType::Unknown; }
+
 // FusedConv with a paired 1x1 convolution: inputs X, W, B, Z, W2, B2 (B, Z
-// and B2 may be omitted) and optionally W packed, outputs Y and Y2.
+// and B2 may be omitted) and optionally W packed or split, outputs Y and Y2.
 void FusedConvPair(const Node& node, const std::string& context, const Views& inputs, const Views& outputs) {
     const int act = ActivationCode(node, context);
     const bool has_bias = inputs[2].dtype != DataType::Unknown;
     const TensorView* z = inputs[3].dtype != DataType::Unknown ? &inputs[3] : nullptr;
     Views main_inputs(inputs.begin(), inputs.begin() + (has_bias ? 3 : 2));
     const ConvCall c = CheckConv(node, context, main_inputs, has_bias, z, Views{outputs[0]});
-    const float* packed = inputs.size() == 7 ? PackedWeights(context, inputs[1], inputs[6], c.d) : nullptr;
+    const float* packed = HasInput(inputs, 6) ? PackedWeights(context, inputs[1], inputs[6], c.d) : nullptr;
     const TensorView& w2 = inputs[4];
     const TensorView& b2 = inputs[5];
     const TensorView& y2 = outputs[1];
@@ -578,7 +599,16 @@ void FusedConvPair(const Node& node, const std::string& context, const Views& in
     if (w2.data == nullptr || y2.data == nullptr || (has_b2 && b2.data == nullptr)) {
         throw InferenceException(context + ": null buffer");
     }
-    if (packed != nullptr) {
+    const float* split = HasInput(inputs, 7) ? SplitWeights(context, inputs[7], d, true) : nullptr;
+    if (split != nullptr) {
+        CheckStatus(nert_hip_conv_presplit_f32(static_cast<const float*>(inputs[0].data),
+                                               static_cast<const float*>(inputs[1].data), split, c.bias, c.residual,
+                                               static_cast<float*>(outputs[0].data),
+                                               static_cast<const float*>(w2.data),
+                                               has_b2 ? static_cast<const float*>(b2.data) : nullptr,
+                                               static_cast<float*>(y2.data), &d, act, Stream()),
+                    context);
+    } else if (packed != nullptr) {
         CheckStatus(nert_hip_conv_packed_f32(static_cast<const float*>(inputs[0].data),
                                              static_cast<const float*>(inputs[1].data), packed, c.bias, c.residual,
                                              static_cast<float*>(outputs[0].data),
@@ -621,23 +651,35 @@ void Conv(const Node& node, const Views& inputs, const Views& outputs) {
 // strides with pad 0, which the runner pairs with a 3x3 pad-1 conv of the
 // same input (a ResNet block's downsampling shortcut): one launch for both
 // (nert_hip_conv_pair_f32). A seventh input is W again in the packed order
-// of nert_hip_conv_packed_f32 (the runner packs 3x3 initializer weights
+// of nert_hip_conv_packed_f32, an eighth W (and W2) split by
+// nert_hip_conv_split_weights (the runner prepares initializer weights
 // once); without a pair, W2 and B2 are then omitted and there is one output.
 void FusedConv(const Node& node, const Views& inputs, const Views& outputs) {
     const std::string context = "FusedConv (node '" + node.name + "')";
-    const bool paired = (inputs.size() == 6 || (inputs.size() == 7 && inputs[4].dtype != DataType::Unknown)) &&
-                        outputs.size() == 2;
+    const bool paired =
+        (inputs.size() == 6 || ((inputs.size() == 7 || inputs.size() == 8) && inputs[4].dtype != DataType::Unknown)) &&
+        outputs.size() == 2;
     if (paired) {
         FusedConvPair(node, context, inputs, outputs);
         return;
     }
-    if (inputs.size() == 7 && outputs.size() == 1 && inputs[4].dtype == DataType::Unknown &&
+    if ((inputs.size() == 7 || inputs.size() == 8) && outputs.size() == 1 && inputs[4].dtype == DataType::Unknown &&
         inputs[5].dtype == DataType::Unknown) {
         const int act = ActivationCode(node, context);
         const bool has_bias = inputs[2].dtype != DataType::Unknown;
         const TensorView* z = inputs[3].dtype != DataType::Unknown ? &inputs[3] : nullptr;
         Views conv_inputs(inputs.begin(), inputs.begin() + (has_bias ? 3 : 2));
         const ConvCall c = CheckConv(node, context, conv_inputs, has_bias, z, outputs);
+        if (HasInput(inputs, 7)) {
+            CheckStatus(nert_hip_conv_presplit_f32(static_cast<const float*>(inputs[0].data),
+                                                   static_cast<const float*>(inputs[1].data),
+                                                   SplitWeights(context, inputs[7], c.d, false), c.bias, c.residual,
+                                                   static_cast<float*>(outputs[0].data), nullptr, nullptr, nullptr,
+                                                   &c.d, act, Stream()),
+                        context);
+            AfterRow(outputs, context);
+            return;
+        }
         const float* packed = PackedWeights(context, inputs[1], inputs[6], c.d);
         CheckStatus(nert_hip_conv_packed_f32(static_cast<const float*>(inputs[0].data),
                                              static_cast<const float*>(inputs[1].data), packed, c.bias, c.residual,

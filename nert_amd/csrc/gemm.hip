@@ -323,11 +323,32 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void GemmKernel(GemmArgs p) {
     constexpr int kBuffer = kOperandLds<Tile::kBM> + kOperandLds<Tile::kBN>;
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[]; // two buffers
     const int64_t tiles_m = (p.m + Tile::kBM - 1) / Tile::kBM;
-    const int64_t tile = GemmTileOrder(blockIdx.x, gridDim.x);
+    int64_t tile;
+    int64_t batch = blockIdx.y;
+    int split = blockIdx.z;
+    int parts = static_cast<int>(gridDim.z);
+    int64_t counter; // of this tile, when it is split
+    if (p.tail_full > 0) {
+        const int id = static_cast<int>(blockIdx.x);
+        int64_t unit;
+        if (id < p.tail_full) {
+            unit = GemmTileOrder(id, p.tail_full);
+            counter = 0;
+        } else {
+            const int q = id - p.tail_full;
+            counter = q / p.tail_pieces;
+            unit = p.tail_full + counter;
+            split = q % p.tail_pieces;
+            parts = p.tail_pieces;
+        }
+        batch = unit / p.tail_tiles;
+        tile = unit % p.tail_tiles;
+    } else {
+        tile = GemmTileOrder(blockIdx.x, gridDim.x);
+        counter = batch * gridDim.x + tile;
+    }
     const int64_t row0 = (tile % tiles_m) * Tile::kBM;
     const int64_t col0 = (tile / tiles_m) * Tile::kBN;
-    const int64_t batch = blockIdx.y;
-    const int split = blockIdx.z;
 
     // Batch offsets from the broadcast strides (innermost axis last).
     int64_t a_off = 0;
@@ -342,7 +363,7 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void GemmKernel(GemmArgs p) {
 
     const int64_t k_begin = static_cast<int64_t>(split) * p.k_per_split;
     int64_t k_end = k_begin + p.k_per_split;
-    if (k_end > p.k) {
+    if (k_end > p.k || (p.tail_full > 0 && parts == 1)) {
         k_end = p.k;
     }
 
@@ -471,10 +492,9 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void GemmKernel(GemmArgs p) {
     }
 
     const int64_t plane = p.m * p.n;
-    if (p.counters != nullptr) {
-        const int64_t t = batch * gridDim.x + tile;
-        float* slots = p.split_slots + t * gridDim.z * Tile::kBM * Tile::kBN;
-        if (FinishSplitParts<RB, CB, T, double>(acc, slots, p.counters + t, split, static_cast<int>(gridDim.z),
+    if (p.counters != nullptr && parts > 1) {
+        float* slots = p.split_slots + counter * parts * Tile::kBM * Tile::kBN;
+        if (FinishSplitParts<RB, CB, T, double>(acc, slots, p.counters + counter, split, parts,
                                                 reinterpret_cast<int*>(lds))) {
             GemmEpilogue<Tile>(p, acc, p.y + batch * plane, row0 + wave_row, col0 + wave_col, true);
         }
@@ -664,7 +684,13 @@ template <class Tile, class Offset = uint32_t>
 void LaunchShape(GemmArgs p, int64_t batches, int splits, hipStream_t stream) {
     const int64_t tiles = ((p.m + Tile::kBM - 1) / Tile::kBM) * ((p.n + Tile::kBN - 1) / Tile::kBN);
     dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(batches), static_cast<unsigned>(splits));
-    if (p.counters != nullptr) {
+    if (p.tail_full > 0) {
+        const int64_t rest = tiles * batches - p.tail_full;
+        p.tail_tiles = static_cast<int32_t>(tiles);
+        grid = dim3(static_cast<unsigned>(p.tail_full + rest * p.tail_pieces), 1, 1);
+        p.split_slots = static_cast<float*>(
+            Workspace(rest * p.tail_pieces * Tile::kBM * Tile::kBN * static_cast<int64_t>(sizeof(float)), stream));
+    } else if (p.counters != nullptr) {
         p.split_slots = static_cast<float*>(
             Workspace(tiles * batches * splits * Tile::kBM * Tile::kBN * static_cast<int64_t>(sizeof(float)), stream));
     }
@@ -703,9 +729,37 @@ bool NarrowOperands(const GemmArgs& p) {
     return a && b;
 }
 
+void LaunchTile(const GemmArgs& p, int64_t batches, int shape, bool narrow, int splits, hipStream_t stream) {
+    switch (shape) {
+    case 0:
+        LaunchShape<TileL>(p, batches, splits, stream);
+        break;
+    case 1:
+        LaunchShape<TileM>(p, batches, splits, stream);
+        break;
+    case 3:
+        LaunchShape<TileN>(p, batches, splits, stream);
+        break;
+    case 4:
+        LaunchShape<TileX>(p, batches, splits, stream);
+        break;
+    case 5:
+        narrow ? LaunchShape<TileQ>(p, batches, splits, stream)
+               : LaunchShape<TileQ, int64_t>(p, batches, splits, stream);
+        break;
+    default:
+        LaunchShape<TileS>(p, batches, splits, stream);
+        break;
+    }
+}
+
 // One configuration: tile shape (0 L, 1 M, 2 S, 3 N, 4 X, 5 Q) and split-K count
-// (0: the PlanSplits choice for that shape).
-void LaunchConfig(GemmArgs p, int64_t batches, int shape, int force_splits, hipStream_t stream) {
+// (0: the PlanSplits choice for that shape; kTailSplit: only the tiles of the
+// last, partly empty round of workgroups are split). False when there is no
+// such round.
+constexpr int kTailSplit = -1;
+
+bool LaunchConfig(GemmArgs p, int64_t batches, int shape, int force_splits, hipStream_t stream) {
     const bool narrow = NarrowOperands(p);
     if (!narrow) {
         shape = 5;
@@ -736,9 +790,40 @@ void LaunchConfig(GemmArgs p, int64_t batches, int shape, int force_splits, hipS
         break;
     }
     const int64_t k_tiles = (p.k + bk - 1) / bk;
-    int splits = force_splits > 0
+    int splits = force_splits > 0 // (kTailSplit returns below)
                      ? static_cast<int>(std::min<int64_t>(force_splits, std::max<int64_t>(k_tiles, 1)))
                      : PlanSplits(tiles, k_tiles, resident, 4, 32);
+    if (force_splits == kTailSplit) {
+        // What the chip holds at once: by LDS (1 to 4 workgroups of a shape
+        // per CU) for all shapes but L and X, which take a CU each. A tile's
+        // pieces keep at least four K steps. On an MI355X the ViT's MLP-up
+        // product (3152 x 3072 x 768, 312 tiles of 256 x 128 on 256 CUs)
+        // otherwise spends half its time in a round of 56 tiles.
+        constexpr int64_t kHeld[6] = {256, 512, 1024, 512, 256, 768};
+        const int64_t held = kHeld[shape];
+        const int64_t rest = tiles % held;
+        if (tiles <= held || rest == 0 || tiles >= (int64_t{1} << 26)) {
+            return false;
+        }
+        int pieces = 1;
+        double round = 1.0;
+        for (int q = 2; q <= std::min<int64_t>(k_tiles / 4, 16); ++q) {
+            const double r = std::ceil(static_cast<double>(rest * q) / static_cast<double>(held)) / q;
+            if (r < round - 1e-9) {
+                round = r;
+                pieces = q;
+            }
+        }
+        if (pieces == 1 || (p.counters = TileCounters(rest)) == nullptr) {
+            return false;
+        }
+        p.k_per_split = ((k_tiles + pieces - 1) / pieces) * bk;
+        p.tail_pieces = static_cast<int32_t>((k_tiles * bk + p.k_per_split - 1) / p.k_per_split);
+        p.tail_full = static_cast<int32_t>(tiles - rest);
+        p.partial = nullptr;
+        LaunchTile(p, batches, shape, narrow, 1, stream);
+        return true;
+    }
     p.k_per_split = ((k_tiles + splits - 1) / splits) * bk;
     if (p.k == 0) {
         p.k_per_split = 0;
@@ -756,27 +841,7 @@ void LaunchConfig(GemmArgs p, int64_t batches, int shape, int force_splits, hipS
                 static_cast<float*>(Workspace(static_cast<int64_t>(splits) * batches * p.m * p.n * 4, stream));
         }
     }
-    switch (shape) {
-    case 0:
-        LaunchShape<TileL>(p, batches, splits, stream);
-        break;
-    case 1:
-        LaunchShape<TileM>(p, batches, splits, stream);
-        break;
-    case 3:
-        LaunchShape<TileN>(p, batches, splits, stream);
-        break;
-    case 4:
-        LaunchShape<TileX>(p, batches, splits, stream);
-        break;
-    case 5:
-        narrow ? LaunchShape<TileQ>(p, batches, splits, stream)
-               : LaunchShape<TileQ, int64_t>(p, batches, splits, stream);
-        break;
-    default:
-        LaunchShape<TileS>(p, batches, splits, stream);
-        break;
-    }
+    LaunchTile(p, batches, shape, narrow, splits, stream);
     if (splits > 1 && p.counters == nullptr) {
         const int vec = p.n % 4 == 0 ? 4 : 1;
         const int64_t total = batches * p.m * p.n;
@@ -790,23 +855,26 @@ void LaunchConfig(GemmArgs p, int64_t batches, int shape, int force_splits, hipS
         }
         CheckLaunch("SplitReduceKernel launch");
     }
+    return true;
 }
 
 // Candidates: 0-11 shape i / 4 (L, M, S) with split count {PlanSplits, 1,
 // 2, 4}[i % 4]; 12 the skinny kernel; 13-24 shape 3 + (i - 13) / 4 (N, X,
-// Q) with split count {...}[(i - 13) % 4].
+// Q) with split count {...}[(i - 13) % 4]; 25-30 shape i - 25 with the tail split.
 using GemmKey = std::array<int64_t, 10>;
 constexpr int kGemmSplits[4] = {0, 1, 2, 4};
-constexpr int kGemmCandidates = 25;
+constexpr int kGemmCandidates = 31;
 constexpr int kSkinnyCandidate = 12;
 
-void LaunchTiled(const GemmArgs& p, int64_t batches, int i, hipStream_t stream) {
-    if (i < kSkinnyCandidate) {
-        LaunchConfig(p, batches, i / 4, kGemmSplits[i % 4], stream);
-    } else {
-        LaunchConfig(p, batches, 3 + (i - kSkinnyCandidate - 1) / 4, kGemmSplits[(i - kSkinnyCandidate - 1) % 4],
-                     stream);
+bool LaunchTiled(const GemmArgs& p, int64_t batches, int i, hipStream_t stream) {
+    if (i >= 25) {
+        return LaunchConfig(p, batches, i - 25, kTailSplit, stream);
     }
+    if (i < kSkinnyCandidate) {
+        return LaunchConfig(p, batches, i / 4, kGemmSplits[i % 4], stream);
+    }
+    return LaunchConfig(p, batches, 3 + (i - kSkinnyCandidate - 1) / 4, kGemmSplits[(i - kSkinnyCandidate - 1) % 4],
+                        stream);
 }
 
 } // namespace
@@ -845,8 +913,7 @@ void LaunchGemm(GemmArgs p, int64_t batches, hipStream_t stream) {
             LaunchSkinny(p, stream);
             return;
         }
-        if (i >= 0 && i < kGemmCandidates && i != kSkinnyCandidate) {
-            LaunchTiled(p, batches, i, stream);
+        if (i >= 0 && i < kGemmCandidates && i != kSkinnyCandidate && LaunchTiled(p, batches, i, stream)) {
             return;
         }
     }
@@ -861,8 +928,7 @@ void LaunchGemm(GemmArgs p, int64_t batches, hipStream_t stream) {
                                        LaunchSkinny(q, stream);
                                        return true;
                                    }
-                                   LaunchTiled(q, batches, i, stream);
-                                   return true;
+                                   return LaunchTiled(q, batches, i, stream);
                                });
     if (c == kSkinnyCandidate && skinny) {
         LaunchSkinny(p, stream);
@@ -870,7 +936,9 @@ void LaunchGemm(GemmArgs p, int64_t batches, hipStream_t stream) {
     }
     // (A cached skinny choice with operands that lost its alignment takes
     // the fallback tiles.)
-    LaunchTiled(p, batches, c == kSkinnyCandidate ? fallback : c, stream);
+    if (!LaunchTiled(p, batches, c == kSkinnyCandidate ? fallback : c, stream)) {
+        LaunchTiled(p, batches, fallback, stream);
+    }
 }
 
 } // namespace nert_hip

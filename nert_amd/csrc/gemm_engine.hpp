@@ -29,6 +29,13 @@ struct GemmArgs {
     // slots [batch * tiles + tile][split][BM * BN].
     uint32_t* counters;
     float* split_slots;
+    // Set by LaunchGemm: > 0 when only the last tiles are split along K.
+    // Workgroups [0, tail_full) take a tile whole, the rest are the
+    // `tail_pieces` parts of the other tiles; a tile number runs over the
+    // batches, `tail_tiles` tiles each.
+    int32_t tail_full;
+    int32_t tail_pieces;
+    int32_t tail_tiles;
     // Optional activation after the bias (fused MatMul rows): act 1 is the
     // erf Gelu chain y -> y * (erf(y / act_div) + act_add) * act_mul.
     int act;

@@ -81,6 +81,11 @@ hipStream_t DefaultStream() {
     return Ctx().stream;
 }
 
+bool WorkspaceHolds(int64_t bytes, int slot) {
+    EnsureReady();
+    return slot >= 0 && slot < kWorkspaceSlots && bytes <= Ctx().workspace_bytes[slot];
+}
+
 void* Workspace(int64_t bytes, hipStream_t stream, int slot) {
     EnsureReady();
     if (slot < 0 || slot >= kWorkspaceSlots) {

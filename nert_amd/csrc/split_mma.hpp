@@ -133,6 +133,20 @@ struct SplitAccum {
         }
     }
 
+    // The same for columns j and j + 1 alone.
+    __device__ __forceinline__ void StepPair(int i, int j, const nert_uintx4 (&row)[3], const nert_uintx4 (&col)[CB][3]) {
+        constexpr int kCol[6] = {1, 2, 0, 1, 0, 0};
+        constexpr int kRow[6] = {1, 0, 2, 0, 1, 0};
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                nert_floatx4& sum = t < 5 ? small[i][j + d] : big[i][j + d];
+                sum = MfmaBf16(col[j + d][kCol[t]], row[kRow[t]], sum);
+            }
+        }
+    }
+
     // Adds the two sets and undoes the scaling, in `big`; true (to the whole
     // wave) when some sum is not finite and the block has to be computed
     // again in float32.

@@ -21,6 +21,7 @@ before the split axis has extent 1): each part is the input at a byte offset.
 from __future__ import annotations
 
 import ctypes as C
+import dataclasses
 from typing import Any, Iterable
 
 import numpy as np
@@ -282,9 +283,10 @@ def pair_downsample_convs(g: Graph) -> Graph:
     return Graph(nodes=nodes, initializers=g.initializers, inputs=g.inputs, outputs=g.outputs, tensors=g.tensors)
 
 
-def pack_conv_weights(g: Graph) -> Graph:
+def pack_conv_weights(g: Graph, split: bool = False) -> Graph:
     """Gives every 3x3 Conv or FusedConv whose weight is a float32
-    initializer with C/group a multiple of 8 a second copy of that weight in
+    initializer with C/group a multiple of 8 (with `split`, unless the
+    split-operand kernel always runs it: stride 1, C/group >= 32) a second copy of that weight in
     the order the 3x3 LDS-patch kernel stores it -- per output channel,
     blocks of 8 input channels, in a block the 9 taps, in a tap the 8
     channels: packed[m][b][t][j] = W[m][8 b + j][t] -- as the FusedConv row's
@@ -299,7 +301,8 @@ def pack_conv_weights(g: Graph) -> Graph:
         w_name = n.inputs[1] if len(n.inputs) > 1 else ""
         w = g.initializers.get(w_name)
         fits = n.op in ("Conv", "FusedConv") and len(n.inputs) <= 6 and w is not None and w.dtype == np.float32 and \
-            w.ndim == 4 and w.shape[2:] == (3, 3) and w.shape[1] % 8 == 0
+            w.ndim == 4 and w.shape[2:] == (3, 3) and w.shape[1] % 8 == 0 and \
+            not (split and w.shape[1] >= 32 and set(n.attrs.get("strides", [1])) == {1})
         if not fits:
             nodes.append(n)
             continue
@@ -312,6 +315,55 @@ def pack_conv_weights(g: Graph) -> Graph:
         ins = list(n.inputs) + [""] * (6 - len(n.inputs)) + [name]
         nodes.append(Node("FusedConv", ins, list(n.outputs), dict(n.attrs), n.name))
     return Graph(nodes=nodes, initializers=initializers, inputs=g.inputs, outputs=g.outputs, tensors=tensors)
+
+
+@dataclasses.dataclass
+class SplitWeights:
+    """Convolution weights a Program splits once on the device
+    (nert_hip_conv_split_weights): `parts` are (weight, taps), one behind the
+    other in the tensor `name`."""
+    name: str
+    parts: list[tuple[str, int]]
+    channels: int  # per group
+    outputs: int
+    group: int
+
+    def words(self) -> list[int]:
+        """Size of every part: per group, 16 rows x 32 channels at a time,
+        three bf16 pieces."""
+        rows = self.group * -(-(self.outputs // self.group) // 16)
+        return [rows * -(-self.channels // 32) * taps * 768 for _, taps in self.parts]
+
+
+def split_conv_weights(g: Graph) -> tuple[Graph, list[SplitWeights]]:
+    """Gives every Conv or FusedConv that the split-operand kernel takes (3x3,
+    or 1x1 with a stride; at least 16 channels per group, a multiple of 8)
+    and whose weights are float32 initializers the split copy of them as the
+    FusedConv row's eighth input, which nert_hip_conv_presplit_f32 copies to
+    LDS instead of splitting every tile's weights again. Returns the graph
+    and what to split. The results are bit-identical."""
+    tensors = dict(g.tensors)
+    nodes: list[Node] = []
+    wanted: dict[str, SplitWeights] = {}
+    for n in g.nodes:
+        geo = _conv_geometry(g, n) if len(n.inputs) <= 7 else None
+        w = g.initializers.get(n.inputs[1]) if geo is not None else None
+        w2 = n.inputs[4] if len(n.inputs) > 4 else ""
+        fits = w is not None and w.dtype == np.float32 and w.ndim == 4 and w.shape[1] >= 16 and \
+            w.shape[1] % 8 == 0 and geo[4] > 0 and w.shape[0] > 0 and w.shape[0] % geo[4] == 0 and \
+            (not w2 or (w2 in g.initializers and g.initializers[w2].dtype == np.float32)) and \
+            (w.shape[2:] == (3, 3) or (w.shape[2:] == (1, 1) and list(geo[1]) != [1, 1]))
+        if not fits:
+            nodes.append(n)
+            continue
+        parts = [(n.inputs[1], w.shape[2] * w.shape[3])] + ([(w2, 1)] if w2 else [])
+        s = SplitWeights(":".join(p for p, _ in parts) + ":split", parts, w.shape[1], w.shape[0], geo[4])
+        wanted.setdefault(s.name, s)
+        tensors[s.name] = (np.dtype(np.float32), (sum(s.words()),))
+        nodes.append(Node("FusedConv", (list(n.inputs) + [""] * 7)[:7] + [s.name], list(n.outputs), dict(n.attrs),
+                          n.name))
+    return Graph(nodes=nodes, initializers=g.initializers, inputs=g.inputs, outputs=g.outputs, tensors=tensors), \
+        list(wanted.values())
 
 
 def _scalar(g: Graph, name: str) -> float | None:
@@ -634,7 +686,7 @@ def fuse_rows(g: Graph, attention: bool = True, pairs: bool = True, packed: bool
     if pairs:
         g = pair_downsample_convs(g)
     if packed:
-        g = pack_conv_weights(g)
+        g = pack_conv_weights(g, split=True)
     if attention:
         g = fuse_attention(g)
     return fuse_add_layernorm(fuse_matmul_chains(g))
@@ -645,6 +697,9 @@ class Program:
                  packed: bool = True):
         if fuse:
             g = fuse_rows(g, attention, pairs, packed)
+        splits: list[SplitWeights] = []
+        if fuse and packed:
+            g, splits = split_conv_weights(g)
         self.alias: dict[str, tuple[str, int]] = {}
         if views:
             g, self.alias = alias_views(g)
@@ -654,6 +709,13 @@ class Program:
         self.resident: dict[str, DeviceArray] = {}
         for name, value in g.initializers.items():
             self.resident[name] = DeviceArray.from_host(value)
+        for s in splits:
+            out = self.resident[s.name] = DeviceArray((sum(s.words()),), np.float32)
+            at = out.ptr
+            for (weight, taps), words in zip(s.parts, s.words()):
+                check(lib().nert_hip_conv_split_weights(self.resident[weight].ptr, at, s.outputs, s.channels, taps,
+                                                        s.group, None), "split weights")
+                at += 4 * words
         for name in g.inputs:
             dtype, shape = g.tensors[name]
             self.resident[name] = DeviceArray(shape, dtype)

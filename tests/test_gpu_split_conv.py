@@ -1,0 +1,136 @@
+"""The split-operand convolution (nert_amd/csrc/conv_split.hip) against
+float64: every tile shape and way of cutting tiles, at widths, channel counts
+and strides on both sides of its patch and block edges."""
+
+import numpy as np
+import pytest
+
+from nert_amd.device import DeviceArray, check, lib, run_node
+from nert_amd.graph import Graph
+from nert_amd.runner import Program
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+def _conv64(x, w, b, s, p, d, g):
+    """Convolution in float64, tap by tap."""
+    n, c, h, wd = x.shape
+    m, cg, kh, kw = w.shape
+    oh, ow = (h + 2 * p - d * (kh - 1) - 1) // s + 1, (wd + 2 * p - d * (kw - 1) - 1) // s + 1
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (p, p), (p, p))).reshape(n, g, cg, h + 2 * p, wd + 2 * p)
+    wg = w.astype(np.float64).reshape(g, m // g, cg, kh, kw)
+    y = np.zeros((n, g, m // g, oh, ow))
+    for r in range(kh):
+        for q in range(kw):
+            tap = xp[:, :, :, r * d:r * d + s * (oh - 1) + 1:s, q * d:q * d + s * (ow - 1) + 1:s]
+            y += np.einsum("gmc,ngchw->ngmhw", wg[..., r, q], tap)
+    return y.reshape(n, m, oh, ow) + b.reshape(1, m, 1, 1)
+
+
+def _split(parts, m, cg, g):
+    """The split copies of `parts`, one behind the other."""
+    words = [lib().nert_hip_conv_split_words(m, cg, v.shape[2] * v.shape[3], g) for v in parts]
+    out = DeviceArray((sum(words),), F)
+    at = out.ptr
+    keep = [DeviceArray.from_host(v) for v in parts]
+    for v, dv, n in zip(parts, keep, words):
+        check(lib().nert_hip_conv_split_weights(dv.ptr, at, m, cg, v.shape[2] * v.shape[3], g, None), "split")
+        at += 4 * n
+    check(lib().nert_hip_stream_sync(None), "sync")
+    return out
+
+
+def _bound(x, w, b, s, p, d, g):
+    """Two accumulators round once per K step of 32 (a step truncates, so a
+    whole ulp, 2^-23, of the products' sizes), the left-out products are
+    below 2^-25, bias and last additions three more roundings."""
+    steps = w.shape[2] * w.shape[3] * -(-w.shape[1] // 32)
+    return (2 * steps + 8) * 2.0 ** -23 * _conv64(np.abs(x), np.abs(w), np.abs(b), s, p, d, g)
+
+
+# x shape, outputs, kernel, stride, pad, dilation, group
+CASES = [((2, 64, 20, 20), 64, 3, 1, 1, 1, 1), ((3, 32, 15, 13), 48, 3, 2, 1, 1, 1), ((1, 16, 9, 9), 32, 3, 1, 1, 1, 1),
+         ((2, 64, 12, 12), 48, 3, 1, 1, 1, 2), ((5, 64, 57, 57), 128, 3, 2, 1, 1, 1), ((1, 40, 5, 112), 96, 3, 1, 1, 1, 1),
+         ((33, 64, 7, 7), 72, 3, 1, 1, 1, 1), ((2, 24, 19, 23), 40, 3, 1, 2, 2, 1), ((2, 24, 19, 23), 40, 3, 2, 2, 3, 1),
+         ((1, 512, 8, 8), 512, 3, 1, 0, 1, 1), ((2, 64, 56, 56), 128, 1, 2, 0, 1, 1), ((3, 40, 14, 14), 200, 1, 3, 1, 1, 1)]
+
+
+@pytest.mark.parametrize("xs,m,k,s,p,d,g", CASES)
+def test_split_conv_every_candidate(gpu, monkeypatch, xs, m, k, s, p, d, g):
+    rng = np.random.default_rng(xs[1] * m + s)
+    x = rng.standard_normal(xs).astype(F)
+    w = (rng.standard_normal((m, xs[1] // g, k, k)) / np.sqrt(xs[1] // g * k * k)).astype(F)
+    b = rng.standard_normal(m).astype(F)
+    want, bound = _conv64(x, w, b, s, p, d, g), _bound(x, w, b, s, p, d, g)
+    z = rng.standard_normal(want.shape).astype(F)
+    w2 = (rng.standard_normal((m, xs[1], 1, 1)) / np.sqrt(xs[1])).astype(F)
+    attrs = {"kernel_shape": [k, k], "strides": [s, s], "pads": [p] * 4, "dilations": [d, d], "group": g}
+    dx, dw, db, dz, dw2 = (DeviceArray.from_host(v) for v in (x, w, b, z, w2))
+    split = _split([w], m, xs[1] // g, g)
+    pair = k == 3 and p == 1 and d == 1 and g == 1
+    for cand in range(400, 421):
+        monkeypatch.setenv("NERT_HIP_CONV_CANDIDATE", str(cand))
+
+        def run(ins, outputs=1, act=None):
+            ys = [DeviceArray(want.shape, F) for _ in range(outputs)]
+            run_node("FusedConv", ins, ys, dict(attrs, activation=act) if act else attrs)
+            return [y.to_host() for y in ys]
+
+        y = run([dx, dw, db])[0]
+        assert np.all(np.abs(y - want) <= bound), cand
+        # weights split once or per call, and the epilogue: the same bits
+        assert np.array_equal(run([dx, dw, db, None, None, None, None, split])[0], y), cand
+        assert np.array_equal(run([dx, dw, db, dz], act="Relu")[0], np.maximum(y + z, F(0))), cand
+        if pair:
+            y1, y2 = run([dx, dw, db, None, dw2, db], 2)
+            assert np.array_equal(y1, y), cand
+            assert np.all(np.abs(y2 - _conv64(x, w2, b, s, 0, 1, 1)) <= _bound(x, w2, b, s, 0, 1, 1)), cand
+            both = _split([w, w2], m, xs[1], 1)
+            z1, z2 = run([dx, dw, db, None, dw2, db, None, both], 2)
+            assert np.array_equal(z1, y) and np.array_equal(z2, y2), cand
+
+
+@pytest.mark.parametrize("cand", [400, 403, 407, 409, 418])
+def test_split_conv_special_values(gpu, monkeypatch, cand):
+    """An infinite, NaN, huge or subnormal input reaches exactly the outputs
+    whose windows hold it, as in float32; the others keep their values."""
+    monkeypatch.setenv("NERT_HIP_CONV_CANDIDATE", str(cand))
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((4, 64, 14, 14)).astype(F)
+    x[0, 3, 5, 6], x[0, 7, 11, 2], x[1, 0, 0, 0] = np.inf, -np.inf, np.nan
+    x[2] *= F(1e33)
+    x[3] *= F(1e-39)
+    w = (rng.standard_normal((64, 64, 3, 3)) * 0.05).astype(F)
+    b = np.zeros(64, F)
+    y = DeviceArray((4, 64, 14, 14), F)
+    run_node("Conv", [DeviceArray.from_host(v) for v in (x, w, b)], [y], {"pads": [1, 1, 1, 1]})
+    y = y.to_host()
+    with np.errstate(all="ignore"):
+        want = _conv64(x, w, b, 1, 1, 1, 1)
+        bound = _bound(np.where(np.isfinite(x), x, 0), w, b, 1, 1, 1, 1) + 2.0 ** -149 * 40
+    finite = np.isfinite(want)
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(y[~finite & ~np.isnan(want)],
+                                                                          want[~finite & ~np.isnan(want)])
+    assert np.all(np.abs(y - want)[finite] <= bound[finite])
+
+
+def test_program_splits_weights_once(gpu):
+    """A Program's split weights change no bit against the separate rows."""
+    rng = np.random.default_rng(9)
+    g = Graph()
+    x = g.add_input("x", F, (2, 48, 17, 17))
+    w = g.add_initializer("w", (rng.standard_normal((40, 48, 3, 3)) * 0.05).astype(F))
+    v = g.add_initializer("v", (rng.standard_normal((64, 40, 3, 3)) * 0.05).astype(F))
+    (a,) = g.add_node("Conv", [x, w], [("a", F, (2, 40, 17, 17))], {"pads": [1, 1, 1, 1]})
+    (c,) = g.add_node("Conv", [a, v], [("c", F, (2, 64, 9, 9))], {"pads": [1, 1, 1, 1], "strides": [2, 2]})
+    g.outputs = [a, c]
+    data = rng.standard_normal((2, 48, 17, 17)).astype(F)
+    outs = []
+    for fuse in (False, True):
+        prog = Program(g, fuse=fuse)
+        prog.set_input("x", data)
+        prog.run()
+        outs.append([prog.output(o) for o in g.outputs])
+        prog.close()
+    assert all(np.array_equal(p, q) for p, q in zip(*outs))
