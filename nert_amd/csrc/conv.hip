@@ -2550,24 +2550,12 @@ bool TrySmallChannelConv(const ConvArgs& p, hipStream_t stream) {
     return LaunchSmallCandidate(c, p, stream) || LaunchSmallCandidate(1, p, stream);
 }
 
-// y = act(y + residual) in place: the fused pointwise convolution's
-// epilogue, run after the GEMM has written conv + bias (each step rounded
-// like the Add and activation rows).
-__global__ void ResidualActKernel(float* y, const float* residual, int act, int64_t n) {
-    for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        float v = y[i];
-        if (residual != nullptr) {
-            v = __fadd_rn(v, residual[i]);
-        }
-        y[i] = Activate(act, v);
-    }
-}
-
 // A 1x1, stride-1, unpadded, ungrouped convolution is Y[b] = W[M,C] * X[b][C,P]
 // with P = D*H*W: a batched GEMM whose B batches are the images. The fused
-// form (residual, activation) runs the same GEMM and then ResidualActKernel, so a
-// Conv and a FusedConv of one geometry sum in the same order.
+// form (residual, activation) is the same GEMM with that in its epilogue, so a
+// Conv and a FusedConv of one geometry sum in the same order. (As a pass of
+// its own it took 8 of 82 us of a detector neck level, 8 x 192 -> 64 channels
+// at 80 x 80.)
 // ---- Non-overlapping patches (stride = kernel, no padding): a GEMM -----------
 //
 // A conv whose windows tile the input exactly (the ViT patch embedding:
@@ -2637,6 +2625,8 @@ bool TryPatchGemm(const ConvArgs& p, hipStream_t stream) {
     g.bias = p.bias;
     g.bias_sm = 1;
     g.bias_sn = 0;
+    g.residual = p.residual;
+    g.conv_act = p.act;
     if (p.plane_out % 4 == 0 && p.n_total < (int64_t{1} << 31) &&
         p.batch * p.c * p.plane_in < (int64_t{1} << 31)) {
         // One GEMM over every image's patches (N = batch x pixels, no
@@ -2678,11 +2668,6 @@ bool TryPatchGemm(const ConvArgs& p, hipStream_t stream) {
         g.b_bs[0] = p.plane_out * k_total;
         LaunchGemm(g, p.batch, stream);
     }
-    if (p.residual != nullptr || p.act != 0) {
-        const int64_t n = p.batch * p.m * p.plane_out;
-        ResidualActKernel<<<GridFor(n, 256, 16384), 256, 0, stream>>>(p.y, p.residual, p.act, n);
-        CheckLaunch("ResidualActKernel launch");
-    }
     return true;
 }
 
@@ -2709,16 +2694,13 @@ bool TryPointwise(const ConvArgs& p, hipStream_t stream) {
     g.bias = p.bias;
     g.bias_sm = 1;
     g.bias_sn = 0;
+    g.residual = p.residual;
+    g.conv_act = p.act;
     g.batch_rank = 1;
     g.bdims[0] = p.batch;
     g.a_bs[0] = 0;
     g.b_bs[0] = p.c * p.plane_in;
     LaunchGemm(g, p.batch, stream);
-    if (p.residual != nullptr || p.act != 0) {
-        const int64_t n = p.batch * p.m * p.plane_out;
-        ResidualActKernel<<<GridFor(n, 256, 16384), 256, 0, stream>>>(p.y, p.residual, p.act, n);
-        CheckLaunch("ResidualActKernel launch");
-    }
     return true;
 }
 
@@ -2784,13 +2766,16 @@ ConvArgs MakeConvArgs(const float* x, const float* w, const float* bias, const f
     return p;
 }
 
-// Split-operand kernel (0) or fp32 kernels (1). With stride 1 and at least 32
-// channels per group the split one is ahead throughout (ResNet-18 bs32 layers
-// 51-57 us against 70-74 on an MI355X). With a stride a patch is two to four
-// times the pixels for the same products, and below 32 channels half of each
-// K step is zeros: there the lead changes with the geometry (64 -> 128
-// channels at 57 x 57, batch 5: 20.3 against 18 us; 64 -> 128 at 56 x 56,
-// batch 32: 37 against 44), and the two are timed.
+// Split-operand kernel (0) or fp32 kernels (1). With stride 1, at least 32
+// channels per group and 2^31 or more products the split one is ahead
+// throughout (ResNet-18 bs32 layers, 3.7e9 products: 51-57 us against 70-74
+// on an MI355X). With a stride a patch is two to four times the pixels for
+// the same products, below 32 channels half of each K step is zeros, and a
+// small problem runs a few workgroups whose steps wait for their loads:
+// there the lead changes with the geometry (stride 2, 64 -> 128 channels at
+// 57 x 57, batch 5: 19.3 against 17.4 us; at 56 x 56, batch 32: 37 against
+// 45.6; 16 -> 32 at 320 x 320, batch 8: 61.6 against 37.7), and the two are
+// timed.
 template <class Launch>
 int ChoosePath(const char* family, std::map<ConvKey, int>& chosen, const ConvArgs& p, hipStream_t s, Launch launch) {
     if (p.k_h > 3 || p.k_w > 3 || p.cg < 16 || p.cg % 8 != 0) {
@@ -2799,7 +2784,7 @@ int ChoosePath(const char* family, std::map<ConvKey, int>& chosen, const ConvArg
     if (const char* forced = std::getenv("NERT_HIP_CONV_CANDIDATE")) {
         return std::atoi(forced) < 400 ? 1 : 0;
     }
-    if (p.s_h == 1 && p.s_w == 1 && p.cg >= 32) {
+    if (p.s_h == 1 && p.s_w == 1 && p.cg >= 32 && p.m * p.kg * p.n_total >= (int64_t{1} << 31)) {
         return 0;
     }
     return ChooseConvConfig(family, chosen, p, s, 2, 0, launch);

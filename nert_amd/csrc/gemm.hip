@@ -10,6 +10,7 @@
 // the tile counters do not suffice, so the result does not depend on
 // scheduling.
 
+#include "conv_args.hpp"
 #include "gemm_engine.hpp"
 #include "split_mma.hpp"
 #include "tune.hpp"
@@ -239,14 +240,25 @@ __device__ __forceinline__ float FinishWith(const GemmArgs& p, float acc, float 
     return value;
 }
 
-__device__ __forceinline__ float FinishGemm(const GemmArgs& p, float acc, int64_t r, int64_t c) {
-    return FinishWith(p, acc, p.has_bias ? p.bias[r * p.bias_sm + c * p.bias_sn] : 0.0f);
+// A convolution's summand and activation, each rounded as its own row rounds it.
+__device__ __forceinline__ float ConvTail(const GemmArgs& p, float value, int64_t y_index) {
+    if (p.residual != nullptr) {
+        value = __fadd_rn(value, p.residual[y_index]);
+    }
+    return Activate(p.conv_act, value);
+}
+
+// `y_index`: of this output in p.y.
+__device__ __forceinline__ float FinishGemm(const GemmArgs& p, float acc, int64_t r, int64_t c, int64_t y_index) {
+    return ConvTail(p, FinishWith(p, acc, p.has_bias ? p.bias[r * p.bias_sm + c * p.bias_sn] : 0.0f), y_index);
 }
 
 // Writes a wave's sums: raw partial sums (finish = false) or finished outputs.
 // A lane holds four consecutive columns of one row per block, stored as 16
-// bytes when the row pitch and the output allow.
-template <class Tile>
+// bytes when the row pitch and the output allow. TAIL: with the convolution's
+// last steps, in kernels of their own: their branches in the plain epilogue
+// made an 18 us product 24.
+template <class Tile, bool TAIL>
 __device__ __forceinline__ void GemmEpilogue(const GemmArgs& p, const SplitAccum<Tile::kRB, Tile::kCB>& acc,
                                              float* out, int64_t row0, int64_t col0, bool finish) {
     const int lane = threadIdx.x & 63;
@@ -287,6 +299,9 @@ __device__ __forceinline__ void GemmEpilogue(const GemmArgs& p, const SplitAccum
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     value[e] = FinishWith(p, value[e], bias[e]);
+                    if (TAIL && c + e < p.n) {
+                        value[e] = ConvTail(p, value[e], at - p.y + e);
+                    }
                 }
             }
             if (quad) {
@@ -315,7 +330,7 @@ __device__ __forceinline__ int64_t GemmTileOrder(int64_t i, int64_t count) {
 // step of 32 the workgroup splits its BM + BN operand rows into LDS once
 // (global loads of the next step in flight under the MFMAs), then every wave
 // runs 6 kRB kCB MFMAs of 16 x 16 x 32 from it.
-template <class Tile, bool A_KCONTIG, bool B_NCONTIG, bool B_PATCH = false, class Offset = uint32_t>
+template <class Tile, bool A_KCONTIG, bool B_NCONTIG, bool B_PATCH = false, class Offset = uint32_t, bool TAIL = false>
 __global__ __launch_bounds__(Tile::kThreads, 2) void GemmKernel(GemmArgs p) {
     constexpr int RB = Tile::kRB;
     constexpr int CB = Tile::kCB;
@@ -496,13 +511,13 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void GemmKernel(GemmArgs p) {
         float* slots = p.split_slots + counter * parts * Tile::kBM * Tile::kBN;
         if (FinishSplitParts<RB, CB, T, double>(acc, slots, p.counters + counter, split, parts,
                                                 reinterpret_cast<int*>(lds))) {
-            GemmEpilogue<Tile>(p, acc, p.y + batch * plane, row0 + wave_row, col0 + wave_col, true);
+            GemmEpilogue<Tile, TAIL>(p, acc, p.y + batch * plane, row0 + wave_row, col0 + wave_col, true);
         }
         return;
     }
     float* out = p.partial != nullptr ? p.partial + (static_cast<int64_t>(split) * gridDim.y + batch) * plane
                                       : p.y + batch * plane;
-    GemmEpilogue<Tile>(p, acc, out, row0 + wave_row, col0 + wave_col, p.partial == nullptr);
+    GemmEpilogue<Tile, TAIL>(p, acc, out, row0 + wave_row, col0 + wave_col, p.partial == nullptr);
 }
 
 // Sums the split-K partials in split order (deterministic), in double with
@@ -523,7 +538,8 @@ __global__ void SplitReduceKernel(GemmArgs p, int splits, int64_t batches, int v
             for (int s = 1; s < splits; ++s) {
                 sum += p.partial[s * total + i + v];
             }
-            p.y[(i - e) + GemmOutIndex(p, r, c + v)] = FinishGemm(p, static_cast<float>(sum), r, c + v);
+            const int64_t at = (i - e) + GemmOutIndex(p, r, c + v);
+            p.y[at] = FinishGemm(p, static_cast<float>(sum), r, c + v, at);
         }
     }
 }
@@ -564,13 +580,13 @@ __global__ __launch_bounds__(256) void SplitReduceQuadKernel(GemmArgs p, int spl
                 }
             }
         }
+        // Four columns of one output group (groups are whole quads).
+        const int64_t at = p.y_group > 0 ? GemmOutIndex(p, r, 4 * static_cast<int64_t>(cq)) : i;
         nert_floatx4 out;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            out[e] = FinishGemm(p, static_cast<float>(sum[e]), r, 4 * cq + e);
+            out[e] = FinishGemm(p, static_cast<float>(sum[e]), r, 4 * cq + e, at + e);
         }
-        // Four columns of one output group (groups are whole quads).
-        const int64_t at = p.y_group > 0 ? GemmOutIndex(p, r, 4 * static_cast<int64_t>(cq)) : i;
         *reinterpret_cast<nert_floatx4*>(p.y + at) = out;
     }
 }
@@ -640,7 +656,7 @@ __global__ __launch_bounds__(512) void SkinnyGemmKernel(GemmArgs p, int64_t k_sl
     for (int v = 0; v < 16; ++v) {
         const int64_t r = 8 * (v >> 2) + 4 * half + (v & 3);
         if (r < p.m && n_ok) {
-            p.y[r * p.n + n] = FinishGemm(p, acc[v], r, n);
+            p.y[r * p.n + n] = FinishGemm(p, acc[v], r, n, r * p.n + n);
         }
     }
 }
@@ -696,9 +712,21 @@ void LaunchShape(GemmArgs p, int64_t batches, int splits, hipStream_t stream) {
     }
     const bool a_k = p.a_sk == 1;
     const bool b_n = p.b_sn == 1;
+    const bool tail = p.residual != nullptr || p.conv_act != 0;
     if (p.patch.x != nullptr) {
         // (A K-contiguous, one batch: LaunchGemm checks.)
-        LaunchKernel<Tile, GemmKernel<Tile, true, false, true, Offset>>(p, grid, stream);
+        if (tail) {
+            LaunchKernel<Tile, GemmKernel<Tile, true, false, true, Offset, true>>(p, grid, stream);
+        } else {
+            LaunchKernel<Tile, GemmKernel<Tile, true, false, true, Offset>>(p, grid, stream);
+        }
+    } else if (tail) {
+        // (A is a convolution's weights, K-contiguous: LaunchGemm checks.)
+        if (b_n) {
+            LaunchKernel<Tile, GemmKernel<Tile, true, true, false, Offset, true>>(p, grid, stream);
+        } else {
+            LaunchKernel<Tile, GemmKernel<Tile, true, false, false, Offset, true>>(p, grid, stream);
+        }
     } else if (a_k && b_n) {
         LaunchKernel<Tile, GemmKernel<Tile, true, true, false, Offset>>(p, grid, stream);
     } else if (a_k) {
@@ -886,6 +914,9 @@ void LaunchGemm(GemmArgs p, int64_t batches, hipStream_t stream) {
     // Operand strides must make one of each pair unit (contiguous tensors).
     if (!(p.a_sk == 1 || p.a_sm == 1) || !(p.b_sn == 1 || p.b_sk == 1)) {
         throw Error("gemm: operands must be contiguous in one index");
+    }
+    if ((p.residual != nullptr || p.conv_act != 0) && p.a_sk != 1) {
+        throw Error("gemm: a convolution's epilogue needs A K-contiguous");
     }
     if (p.y_group > 0 && (batches != 1 || p.y_group % 4 != 0 || p.n % p.y_group != 0)) {
         throw Error("gemm: grouped output needs one batch and groups of whole quads dividing n");

@@ -40,6 +40,10 @@ struct GemmArgs {
     // erf Gelu chain y -> y * (erf(y / act_div) + act_add) * act_mul.
     int act;
     float act_div, act_add, act_mul;
+    // Optional last steps of a convolution's epilogue: the sum with `residual`
+    // (laid out as y) and the activation (1 Relu, 2 SiLU, as in conv_args.hpp).
+    const float* residual;
+    int conv_act;
     // Output layout (one batch only): 0, Y(m, n) at y[m * n_total + n]; G > 0
     // (a multiple of 4 dividing n), the columns form groups of G stored as
     // [n / G][m][n % G], e.g. a conv's NCHW output when n runs over (image,

@@ -283,10 +283,9 @@ def pair_downsample_convs(g: Graph) -> Graph:
     return Graph(nodes=nodes, initializers=g.initializers, inputs=g.inputs, outputs=g.outputs, tensors=g.tensors)
 
 
-def pack_conv_weights(g: Graph, split: bool = False) -> Graph:
+def pack_conv_weights(g: Graph) -> Graph:
     """Gives every 3x3 Conv or FusedConv whose weight is a float32
-    initializer with C/group a multiple of 8 (with `split`, unless the
-    split-operand kernel always runs it: stride 1, C/group >= 32) a second copy of that weight in
+    initializer with C/group a multiple of 8 a second copy of that weight in
     the order the 3x3 LDS-patch kernel stores it -- per output channel,
     blocks of 8 input channels, in a block the 9 taps, in a tap the 8
     channels: packed[m][b][t][j] = W[m][8 b + j][t] -- as the FusedConv row's
@@ -301,8 +300,7 @@ def pack_conv_weights(g: Graph, split: bool = False) -> Graph:
         w_name = n.inputs[1] if len(n.inputs) > 1 else ""
         w = g.initializers.get(w_name)
         fits = n.op in ("Conv", "FusedConv") and len(n.inputs) <= 6 and w is not None and w.dtype == np.float32 and \
-            w.ndim == 4 and w.shape[2:] == (3, 3) and w.shape[1] % 8 == 0 and \
-            not (split and w.shape[1] >= 32 and set(n.attrs.get("strides", [1])) == {1})
+            w.ndim == 4 and w.shape[2:] == (3, 3) and w.shape[1] % 8 == 0
         if not fits:
             nodes.append(n)
             continue
@@ -686,7 +684,7 @@ def fuse_rows(g: Graph, attention: bool = True, pairs: bool = True, packed: bool
     if pairs:
         g = pair_downsample_convs(g)
     if packed:
-        g = pack_conv_weights(g, split=True)
+        g = pack_conv_weights(g)
     if attention:
         g = fuse_attention(g)
     return fuse_add_layernorm(fuse_matmul_chains(g))

@@ -134,3 +134,28 @@ def test_program_splits_weights_once(gpu):
         outs.append([prog.output(o) for o in g.outputs])
         prog.close()
     assert all(np.array_equal(p, q) for p, q in zip(*outs))
+
+
+@pytest.mark.parametrize("xs,m,k", [((3, 40, 9, 13), 36, 1), ((2, 96, 20, 20), 70, 1), ((2, 8, 16, 16), 40, 4),
+                                    ((2, 8, 12, 20), 40, 4)])
+def test_gemm_conv_epilogue_every_candidate(gpu, monkeypatch, xs, m, k):
+    """The summand and activation of a 1x1 convolution, or of one whose
+    windows tile the input, in the GEMM's epilogue round as the separate rows
+    do, whole tiles and split ones."""
+    rng = np.random.default_rng(m)
+    x = rng.standard_normal(xs).astype(F)
+    w = rng.standard_normal((m, xs[1], k, k)).astype(F)
+    b = rng.standard_normal(m).astype(F)
+    shape = (xs[0], m, xs[2] // k, xs[3] // k)
+    attrs = {"strides": [k, k]}
+    z = rng.standard_normal(shape).astype(F)
+    dx, dw, db, dz = (DeviceArray.from_host(v) for v in (x, w, b, z))
+    y, t, u, fused = (DeviceArray(shape, F) for _ in range(4))
+    for cand in range(31):
+        monkeypatch.setenv("NERT_HIP_GEMM_CANDIDATE", str(cand))
+        run_node("Conv", [dx, dw, db], [y], attrs)
+        run_node("Add", [y, dz], [t])
+        run_node("Sigmoid", [t], [u])
+        run_node("Mul", [t, u], [y])
+        run_node("FusedConv", [dx, dw, db, dz], [fused], dict(attrs, activation="Silu"))
+        assert np.array_equal(fused.to_host(), y.to_host()), cand

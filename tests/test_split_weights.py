@@ -1,0 +1,39 @@
+"""Which convolutions a Program splits weights for, and the size of the copy."""
+
+import numpy as np
+import pytest
+
+from nert_amd import workloads
+from nert_amd.device import lib
+from nert_amd.graph import Graph
+from nert_amd.runner import SplitWeights, fuse_rows, split_conv_weights
+
+F = np.float32
+
+
+@pytest.mark.parametrize("m,cg,group,taps", [(64, 64, 1, [9]), (48, 16, 3, [9]), (33, 40, 1, [1]), (128, 64, 1, [9, 1])])
+def test_words_match_the_library(m, cg, group, taps):
+    s = SplitWeights("s", [(f"w{i}", t) for i, t in enumerate(taps)], cg, m, group)
+    assert s.words() == [lib().nert_hip_conv_split_words(m, cg, t, group) for t in taps]
+
+
+def test_resnet18_splits():
+    """The 16 3x3 convolutions (three with their paired 1x1), not the stem."""
+    g, splits = split_conv_weights(fuse_rows(workloads.resnet18(batch=2)[0]))
+    assert len(splits) == 16 and sum(len(s.parts) == 2 for s in splits) == 3
+    for n in g.nodes:
+        if len(n.inputs) == 8:
+            assert g.tensors[n.inputs[7]] == (np.dtype(F), (sum(next(s for s in splits if s.name == n.inputs[7]).words()),))
+    assert g.nodes[0].op == "FusedConv" and len(g.nodes[0].inputs) < 8
+
+
+@pytest.mark.parametrize("cg,k,stride,fits", [(8, 3, 1, False), (12, 3, 1, False), (16, 3, 1, True), (32, 1, 1, False),
+                                              (32, 1, 2, True), (32, 5, 1, False)])
+def test_rule(cg, k, stride, fits):
+    h = Graph()
+    x = h.add_input("x", F, (1, cg, 9, 9))
+    w = h.add_initializer("w", np.ones((8, cg, k, k), F))
+    out = (9 - k) // stride + 1
+    h.outputs = list(h.add_node("Conv", [x, w], [("y", F, (1, 8, out, out))], {"strides": [stride, stride]}))
+    g, splits = split_conv_weights(h)
+    assert (len(splits) == 1) == fits and (len(g.nodes[0].inputs) == 8) == fits
