@@ -2775,7 +2775,10 @@ ConvArgs MakeConvArgs(const float* x, const float* w, const float* bias, const f
 // there the lead changes with the geometry (stride 2, 64 -> 128 channels at
 // 57 x 57, batch 5: 19.3 against 17.4 us; at 56 x 56, batch 32: 37 against
 // 45.6; 16 -> 32 at 320 x 320, batch 8: 61.6 against 37.7), and the two are
-// timed.
+// timed. The timing launches one convolution over and over, so its weights
+// (split ones are half as many bytes again) stay in the caches; among other
+// layers they do not, and the split kernel must lead by kSplitLead.
+constexpr float kSplitLead = 1.06f;
 template <class Launch>
 int ChoosePath(const char* family, std::map<ConvKey, int>& chosen, const ConvArgs& p, hipStream_t s, Launch launch) {
     if (p.k_h > 3 || p.k_w > 3 || p.cg < 16 || p.cg % 8 != 0) {
@@ -2787,7 +2790,7 @@ int ChoosePath(const char* family, std::map<ConvKey, int>& chosen, const ConvArg
     if (p.s_h == 1 && p.s_w == 1 && p.cg >= 32 && p.m * p.kg * p.n_total >= (int64_t{1} << 31)) {
         return 0;
     }
-    return ChooseConvConfig(family, chosen, p, s, 2, 0, launch);
+    return ChooseConvConfig(family, chosen, p, s, 2, 0, launch, kSplitLead);
 }
 
 // Runs one convolution on the fastest kernel that applies.

@@ -108,14 +108,14 @@ inline ConvKey KeyOf(const ConvArgs& p) {
 
 template <class Launch>
 int ChooseConvConfig(const char* family, std::map<ConvKey, int>& cache, const ConvArgs& p, hipStream_t stream,
-                     int count, int fallback, Launch launch) {
+                     int count, int fallback, Launch launch, float first_weight = 1.0f) {
     static std::mutex mu;
     const size_t y_bytes = static_cast<size_t>(p.batch * p.m * p.plane_out) * sizeof(float);
     return ChooseConfig(family, cache, mu, KeyOf(p), y_bytes, stream, count, fallback, [&](int i, float* scratch) {
         ConvArgs q = p;
         q.y = scratch;
         return launch(i, q, stream);
-    });
+    }, first_weight);
 }
 
 // A 1x1 convolution run with a 3x3 one of the same input, stride and output

@@ -1,4 +1,5 @@
-// Gemm and MatMul on fp32 MFMA (v_mfma_f32_32x32x2_f32).
+// Gemm and MatMul on the bf16 matrix cores with all 24 bits of both operands
+// (split_mma.hpp); few rows (SkinnyGemmKernel) on v_mfma_f32_32x32x2_f32.
 //
 // One kernel serves both rows: Y[b] = alpha * op(A[b]) * op(B[b]) + beta * C,
 // where b runs over up to four broadcast batch axes (MatMul) or is absent

@@ -126,9 +126,11 @@ inline void RecordChoice(const std::string& table_key, int choice,
 
 // launch(i, scratch_y) -> false when candidate i does not fit; it must write
 // its output to scratch_y (scratch_bytes long) instead of the caller's.
+// Candidate 0's times count `first_weight` times.
 template <class Key, class Launch>
 int ChooseConfig(const char* family, std::map<Key, int>& cache, std::mutex& mu, const Key& key,
-                 size_t scratch_bytes, hipStream_t stream, int count, int fallback, Launch launch) {
+                 size_t scratch_bytes, hipStream_t stream, int count, int fallback, Launch launch,
+                 float first_weight = 1.0f) {
     std::lock_guard<std::mutex> lock(mu);
     auto it = cache.find(key);
     if (it != cache.end()) {
@@ -198,7 +200,7 @@ int ChooseConfig(const char* family, std::map<Key, int>& cache, std::mutex& mu, 
                     throw;
                 }
                 Check(hipGraphExecDestroy(exec), "hipGraphExecDestroy");
-                return ms * 1000.0f / static_cast<float>(reps);
+                return ms * 1000.0f / static_cast<float>(reps) * (i == 0 ? first_weight : 1.0f);
             };
             // First pass: one warm eager launch, then a graph of ten launches.
             std::vector<std::pair<float, int>> first;
