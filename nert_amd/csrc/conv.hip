@@ -2777,8 +2777,10 @@ ConvArgs MakeConvArgs(const float* x, const float* w, const float* bias, const f
 // 45.6; 16 -> 32 at 320 x 320, batch 8: 61.6 against 37.7), and the two are
 // timed. The timing launches one convolution over and over, so its weights
 // (split ones are half as many bytes again) stay in the caches; among other
-// layers they do not, and the split kernel must lead by kSplitLead.
-constexpr float kSplitLead = 1.06f;
+// layers they do not (128 -> 128 channels at 29 x 29, batch 5: 20.6 against
+// 22.5 us in its timing, yet no gain in a block of 50), and the split kernel
+// must lead by kSplitLead.
+constexpr float kSplitLead = 1.15f;
 template <class Launch>
 int ChoosePath(const char* family, std::map<ConvKey, int>& chosen, const ConvArgs& p, hipStream_t s, Launch launch) {
     if (p.k_h > 3 || p.k_w > 3 || p.cg < 16 || p.cg % 8 != 0) {
